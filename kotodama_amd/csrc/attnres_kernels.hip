@@ -381,14 +381,17 @@ __device__ __forceinline__ float param_elem(const ParamRaw<VEC>& r, int e, bool 
 
 // Exchange lanes 32..63 of a with lanes 0..31 of b (v_permlane32_swap), and
 // the odd 16-lane rows of a with the even rows of b (v_permlane16_swap).  The
-// leading s_nop covers the VALU-write -> permlane-read hazard.  Inline asm:
+// leading s_nop gives the three wait states that a VALU read of a v_dot2 result
+// needs (the permlane's own hazard after another VALU write takes two); the
+// compiler places neither before inline asm.  With two, sums fed straight from
+// a v_dot2 were read before its last product was in.  Inline asm:
 // this compiler's __builtin_amdgcn_permlane{16,32}_swap return the first
 // register for both results.
 __device__ __forceinline__ void swap_halves32(float& a, float& b) {
-  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  asm volatile("s_nop 2\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
 }
 __device__ __forceinline__ void swap_rows16(float& a, float& b) {
-  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  asm volatile("s_nop 2\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
 }
 
 template <int CTRL, int ROW_MASK>
