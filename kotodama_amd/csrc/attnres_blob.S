@@ -1,4 +1,4 @@
-/* The eleven gfx950 code-object parts, linked into libattnres_hip.so as bytes
+/* The twelve gfx950 code-object parts, linked into libattnres_hip.so as bytes
  * and loaded with hipModuleLoadData.  The build passes -I<dir of the .hsaco>. */
     .section .rodata
     .balign 4096
@@ -45,4 +45,8 @@ attnres_hsaco_part9:
     .global attnres_hsaco_part10
 attnres_hsaco_part10:
     .incbin "attnres_gfx950_part10.hsaco"
+    .balign 4096
+    .global attnres_hsaco_part11
+attnres_hsaco_part11:
+    .incbin "attnres_gfx950_part11.hsaco"
     .section .note.GNU-stack,"",@progbits

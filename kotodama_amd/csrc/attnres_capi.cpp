@@ -34,10 +34,11 @@ extern "C" const unsigned char attnres_hsaco_part7[];
 extern "C" const unsigned char attnres_hsaco_part8[];
 extern "C" const unsigned char attnres_hsaco_part9[];
 extern "C" const unsigned char attnres_hsaco_part10[];
+extern "C" const unsigned char attnres_hsaco_part11[];
 
 namespace {
 
-constexpr int kParts = 11;
+constexpr int kParts = 12;
 constexpr int kMaxDevices = 64;
 constexpr int kMaxThreads = 512;  // __launch_bounds__ of every kernel
 
@@ -108,12 +109,13 @@ struct DeviceState {
   KernelSlot bwd_stream[2 * 10];  // row-per-wave backward: rows of 6 / 8 KiB x S (1..9)
   KernelSlot bwd_add[kBwdFuncs];   // the same with addend rows (_add)
   KernelSlot bwd_stream_add[2 * 10];
+  KernelSlot bwd_rows[3 * 3 * 10];  // narrow rows' backward: plain / _add / _defer x row KiB (1..3) x S (1..9)
   KernelSlot reduce_stage, reduce_cols, reduce_fin;
   KernelSlot merge_bwd[kMergeFuncs];
   KernelSlot bwd_mq[kBwdFuncs];  // batched-query backward: (source, grad_out) dtypes x S x V
   KernelSlot bwd_dqw[4];         // source dtype x V
   KernelSlot bwd_mqg[2 * 9];     // batched-query backward on the matrix cores: query groups x S
-  KernelSlot bwd_defer[4 * 10];  // row-per-wave backward with deferred block gradients: row width x S
+  KernelSlot bwd_defer[2 * 10];  // row-per-wave backward with deferred block gradients: 6 / 8 KiB rows x S
   KernelSlot gather_seg[4 * ATTNRES_SEG_MAX_BLOCKS];  // segment sums: row width x blocks
 };
 
@@ -201,7 +203,7 @@ int ensure_loaded(DeviceState** out) {
       const unsigned char* blobs[kParts] = {attnres_hsaco_part0, attnres_hsaco_part1, attnres_hsaco_part2,
                                             attnres_hsaco_part3, attnres_hsaco_part4, attnres_hsaco_part5,
                                             attnres_hsaco_part6, attnres_hsaco_part7, attnres_hsaco_part8,
-                                            attnres_hsaco_part9, attnres_hsaco_part10};
+                                            attnres_hsaco_part9, attnres_hsaco_part10, attnres_hsaco_part11};
       // On a failure nothing stays half-loaded: the next call starts over.
       auto unload = [&st](int n) {
         for (int j = 0; j < n; ++j) {
@@ -418,9 +420,43 @@ int get_bwd_stream(DeviceState& st, int nch, int s, hipFunction_t* f, bool add =
   return slot_function(st, add ? st.bwd_stream_add[idx] : st.bwd_stream[idx], add ? kBwdStreamAddPart : 4, name, f);
 }
 
+// Row-per-wave backward of narrow rows (code-object part 11): bf16 sources and
+// output gradients, rows of up to 3 KiB of any width, S <= 9 (with addend rows
+// in 3 KiB rows S <= 6: more spill), every row of a token requested at once.
+// AUTO takes it from four rows per CU: at 8192 rows of 1 KiB it measured 1.6-1.8
+// times as fast as the row-per-workgroup kernel, at 2 KiB 1.1-1.5 times, at 3
+// KiB even to 1.2 times; at 1024 rows 1.2 times at every width; at 512 even (3
+// KiB rows at S = 9 4% slower) and at 64 rows of 3 KiB 17% slower.
+constexpr int kBwdRowsPart = 11;
+enum BwdRowsVariant { kBwdRowsPlain = 0, kBwdRowsAdd = 1, kBwdRowsDefer = 2 };
+// Row KiB (rounded up) of that kernel for this call, or 0 for another one.
+int bwd_rows_nch(bool bf, bool gbf, int num_sources, int hidden, int64_t num_tokens, int num_cus, bool add) {
+  if (!bf || !gbf || hidden > 1536 || num_sources < 1 || num_sources > 9) return 0;
+  const int nch = (hidden + 511) / 512;
+  if (add && nch == 3 && num_sources > 6) return 0;
+  if (num_tokens >= (int64_t)1 << 31) return 0;  // 32-bit row counters
+  const int policy = g_policy.load(std::memory_order_relaxed);
+  const int want = policy == ATTNRES_POLICY_STREAM ? 1 : policy == ATTNRES_POLICY_WORKGROUP ? 0 : tuning().stream;
+  return want == 1 || (want < 0 && num_tokens >= 4LL * num_cus) ? nch : 0;
+}
+int get_bwd_rows(DeviceState& st, int nch, int s, BwdRowsVariant var, hipFunction_t* f, int* bpc) {
+  static const char* suffix[] = {"", "_add", "_defer"};
+  char name[96];
+  snprintf(name, sizeof(name), "attnres_route_bwd_rows_c%d_s%d%s", nch, s, suffix[var]);
+  return slot_get(st, st.bwd_rows[((int)var * 3 + nch - 1) * 10 + s], kBwdRowsPart, name,
+                  64 * ATTNRES_BWD_ROWS_WAVES, 0, f, bpc);
+}
+// Its grid: two workgroups per CU where they fit (measured in the kernel's comment).
+int bwd_rows_grid(int64_t num_tokens, int num_cus, int bpc) {
+  const int limit = tuning().bwd_per_cu > 0 ? tuning().bwd_per_cu : 2;
+  const int64_t need = (num_tokens + ATTNRES_BWD_ROWS_WAVES - 1) / ATTNRES_BWD_ROWS_WAVES;
+  const int64_t cap = (int64_t)num_cus * (bpc < limit ? bpc : limit);
+  return (int)(need < cap ? need : cap);
+}
+
 // Deferred block gradients (code-object part 10): the row-per-wave backward
 // forming only the partial's gradient (attnres_route_bwd_stream_c<NCH>_s<S>_defer,
-// S >= 2) and the sums of the blocks' terms
+// S >= 2; rows of 1 and 2 KiB: the _defer kernels above) and the sums of the blocks' terms
 // (attnres_route_bwd_gather_seg_c<NCH>_b<NB>).
 constexpr int kDeferPart = 10;
 // The row widths of the deferred path: hidden 3072, 4096, 1024 and 512 (rows of
@@ -999,6 +1035,12 @@ int attnres_route_bwd_kernel_name(int num_sources, int64_t num_tokens, int hidde
     snprintf(buf, (size_t)buf_len, "attnres_route_bwd_stream_c%d_s%d", nch, num_sources);
     return ATTNRES_OK;
   }
+  const int rnch = bwd_rows_nch(bf, grad_out_dtype == ATTNRES_DTYPE_BF16, num_sources, hidden, num_tokens,
+                                st->num_cus, false);
+  if (rnch > 0) {
+    snprintf(buf, (size_t)buf_len, "attnres_route_bwd_rows_c%d_s%d", rnch, num_sources);
+    return ATTNRES_OK;
+  }
   const int v = bwd_chunks_per_thread(hidden / vec, num_sources, num_tokens, st->num_cus);
   snprintf(buf, (size_t)buf_len, "attnres_route_bwd_%s_g%s_s%d_v%d", bf ? "bf" : "f32",
            grad_out_dtype == ATTNRES_DTYPE_BF16 ? "bf" : "f32", num_sources, v);
@@ -1320,6 +1362,18 @@ static int route_bwd_impl(const void* const* sources, int num_sources, int64_t n
                             grad_out_dtype, grad_out_ld, grad_lse, grad_sources, grad_ld, workspace, workspace_bytes,
                             grad_query, grad_gain, stream, addend);
   }
+  const int rnch = bwd_rows_nch(bf, grad_out_dtype == ATTNRES_DTYPE_BF16, num_sources, hidden, num_tokens,
+                                st->num_cus, add);
+  if (rnch > 0) {
+    hipFunction_t f = nullptr;
+    int bpc = 1;
+    rc = get_bwd_rows(*st, rnch, num_sources, add ? kBwdRowsAdd : kBwdRowsPlain, &f, &bpc);
+    if (rc != ATTNRES_OK) return rc;
+    return route_bwd_finish(f, bwd_rows_grid(num_tokens, st->num_cus, bpc), 64 * ATTNRES_BWD_ROWS_WAVES, 0, *st,
+                            nchunk, sources, num_sources, num_tokens, hidden, src_ld, query, gain, param_dtype, eps,
+                            grad_out, grad_out_dtype, grad_out_ld, grad_lse, grad_sources, grad_ld, workspace,
+                            workspace_bytes, grad_query, grad_gain, stream, addend);
+  }
   const int v = bwd_chunks_per_thread(nchunk, num_sources, num_tokens, st->num_cus);
   const int block = v == 1 ? round64(nchunk) : round64((nchunk + 1) / 2);
   hipFunction_t f = nullptr;
@@ -1404,6 +1458,20 @@ int attnres_route_bwd_defer(const void* const* sources, int num_sources, int64_t
   DeviceState* st = nullptr;
   int rc = ensure_loaded(&st);
   if (rc != ATTNRES_OK) return rc;
+  void* grads[ATTNRES_MAX_SOURCES] = {};
+  const void* adds[ATTNRES_MAX_SOURCES] = {};
+  grads[num_sources - 1] = grad_partial;
+  adds[num_sources - 1] = grad_partial_addend;
+  if (nch <= 2) {
+    hipFunction_t f = nullptr;
+    int bpc = 1;
+    rc = get_bwd_rows(*st, nch, num_sources, kBwdRowsDefer, &f, &bpc);
+    if (rc != ATTNRES_OK) return rc;
+    return route_bwd_finish(f, bwd_rows_grid(num_tokens, st->num_cus, bpc), 64 * ATTNRES_BWD_ROWS_WAVES, 0, *st,
+                            hidden / 8, sources, num_sources, num_tokens, hidden, src_ld, query, gain, param_dtype,
+                            eps, grad_out, grad_out_dtype, grad_out_ld, grad_lse, grads, grad_ld, workspace,
+                            workspace_bytes, grad_query, grad_gain, stream, adds, coef, qfold);
+  }
   if (bwd_stream_lds(nch, num_sources) > (size_t)st->max_lds)
     return fail(ATTNRES_ERR_UNSUPPORTED, "deferred backward: %zu bytes of LDS exceed the device's %d",
                 bwd_stream_lds(nch, num_sources), st->max_lds);
@@ -1411,13 +1479,8 @@ int attnres_route_bwd_defer(const void* const* sources, int num_sources, int64_t
   hipFunction_t f = nullptr;
   rc = get_bwd_defer(*st, nch, num_sources, &f);
   if (rc != ATTNRES_OK) return rc;
-  void* grads[ATTNRES_MAX_SOURCES] = {};
-  const void* adds[ATTNRES_MAX_SOURCES] = {};
-  grads[num_sources - 1] = grad_partial;
-  adds[num_sources - 1] = grad_partial_addend;
   const int64_t need_wg = (num_tokens + kBwdStreamWaves - 1) / kBwdStreamWaves;
-  // rows of 1-2 KiB: more waves per CU to keep the memory system busy
-  const int per_cu = tuning().bwd_per_cu > 0 ? tuning().bwd_per_cu : nch <= 2 ? kBwdMaxPerCu : 1;
+  const int per_cu = tuning().bwd_per_cu > 0 ? tuning().bwd_per_cu : 1;
   const int64_t cap = (int64_t)st->num_cus * per_cu;
   const int grid = (int)(need_wg < cap ? need_wg : cap);
   return route_bwd_finish(f, grid, 64 * kBwdStreamWaves, lds, *st, hidden / 8, sources, num_sources, num_tokens,

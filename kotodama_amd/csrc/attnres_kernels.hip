@@ -206,6 +206,11 @@ __device__ __forceinline__ void st_row_nt(__amdgpu_buffer_rsrc_t r, uint32_t off
   __builtin_amdgcn_raw_buffer_store_b64(v, r, off, 0, 2);
 }
 
+// Non-temporal row load: a row read once.
+__device__ __forceinline__ u32x4 ld_row_nt(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 2);
+}
+
 // Stores hidden from the compiler's wait-count model.  One counter (vmcnt)
 // covers vector loads and stores, and the compiler, which cannot order a
 // pending store against a pending load, waits for a loaded register with
@@ -2383,10 +2388,227 @@ __device__ __forceinline__ void route_bwd_stream_body(const attnres_route_bwd_pa
 }
 
 
-// Non-temporal row load: a row read once.
-__device__ __forceinline__ u32x4 ld_row_nt(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-  return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 2);
+// ------------------------------- row-per-wave backward of narrow rows --
+//
+// The routing backward for bf16 sources and output gradients with rows of up
+// to 3 KiB (any multiple of 8 elements: NCH = the row's KiB, rounded up), one
+// wave per token row.  With so little data per row the kernels above are
+// bound by per-row latency, not by memory: a workgroup per row pays two
+// barriers and an LDS exchange for 1-3 KiB per source, and one row in flight
+// per wave is a serial chain of S + 1 loads.  Here a wave requests the whole
+// token at once (G and the S source rows, up to 30 KiB), reduces its 3S sums
+// with the transposing tree and forms the softmax and the coefficients with
+// lane s for source s, all without a barrier; two 4-wave workgroups per CU
+// overlap one wave's loads with the others' arithmetic and stores (one ran
+// 2-10% slower at 1 KiB rows, four 0-5%).  Per call with the reduction, at 8192
+// rows against a workgroup per row: 1 KiB rows S = 2 26.6 -> 15.0 us, S = 5 41.2
+// -> 23.4, S = 8 54.3 -> 34.2; 1.5 KiB S = 5 48.9 -> 32.4; 2 KiB S = 5 52.7 ->
+// 41.5; 3 KiB S = 5 58.8 -> 57.8, at 32768 rows 252.6 -> 210 (4.2-5.3 TB/s).
+// DEFER at 1 KiB rows, 8192 rows, against route_bwd_stream_body's: S = 2 12.4 ->
+// 11.4 us, S = 5 17.3 -> 15.5.
+// Rows are addressed through buffer resources of the row's bytes, so the
+// chunks past the end of a row that is not whole KiB read zeros and their
+// stores are dropped.  ADD and DEFER as in route_bwd_stream_body.
+template <int S, int NCH, bool ADD = false, bool DEFER = false>
+__device__ __forceinline__ void route_bwd_rows_body(const attnres_route_bwd_params& P) {
+  static_assert(!DEFER || (ADD && S >= 2), "deferred gradients need a committed source and the addend path");
+  constexpr int NV = 3 * S;  // sum(x^2), x.qw, x.G per source
+  constexpr int H2 = (NV + 3) / 4;
+  constexpr int NP = 4 * H2;
+  constexpr int SEG = S <= 8 ? 8 : 16;  // lanes of the softmax
+  constexpr int ROW4 = NCH * 2 * 64;    // float4 slots of one query-gradient row
+  __shared__ float red[ATTNRES_BWD_ROWS_WAVES][NP];
+  __shared__ float4 dq_lds[ATTNRES_BWD_ROWS_WAVES * ROW4];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  // ---- the lane's part of the folded query (zeros past the row end) ----
+  float qw[NCH][8], dq[NCH][8];
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int i = c * 64 + lane;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) qw[c][e] = 0.f, dq[c][e] = 0.f;
+    if (i < P.nchunk) {
+      load_param<8>(P.query, (int64_t)i * 8, P.param_bf16, qw[c]);
+      if (P.gain != nullptr) {
+        float gn[8];
+        load_param<8>(P.gain, (int64_t)i * 8, P.param_bf16, gn);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float prod = qw[c][e] * gn[e];
+          qw[c][e] = P.param_bf16 ? round_bf16(prod) : prod;
+        }
+      }
+      if constexpr (DEFER) {
+        if (blockIdx.x == 0 && wave == 0)
+          stg<u32x4>(static_cast<char*>(P.qfold) + (size_t)i * 16,
+                     u32x4{pack_bf16(qw[c][0], qw[c][1]), pack_bf16(qw[c][2], qw[c][3]),
+                           pack_bf16(qw[c][4], qw[c][5]), pack_bf16(qw[c][6], qw[c][7])});
+      }
+    }
+  }
+
+  // 32-bit wave-uniform row counters (scalar loop control, as in stream_body)
+  const uint32_t n_tok = (uint32_t)P.n_tokens;
+  const uint32_t nw = gridDim.x * ATTNRES_BWD_ROWS_WAVES;
+  const uint32_t row_size = (uint32_t)P.d * 2;
+  const uint32_t lane_off = (uint32_t)lane * 16;
+  auto row_at = [&](const void* base, int64_t ld, uint32_t t) {
+    return row_rsrc(const_cast<char*>(uniform_ptr(reinterpret_cast<uint64_t>(base) + (uint64_t)t * ((uint64_t)ld * 2))),
+                    row_size);
+  };
+  for (uint32_t t = blockIdx.x * ATTNRES_BWD_ROWS_WAVES + (uint32_t)wave; t < n_tok; t += nw) {
+    t = __builtin_amdgcn_readfirstlane(t);
+    // ---- the whole token in one go ----
+    u32x4 x[S][NCH], g[NCH];
+    {
+      const __amdgpu_buffer_rsrc_t gr = row_at(P.grad_out, P.gout_ld, t);
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) g[c] = ld_row_nt(gr, lane_off + (uint32_t)(c * 1024));
+    }
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const __amdgpu_buffer_rsrc_t sr = row_at(P.src[s], P.src_ld, t);
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) x[s][c] = ld_row_nt(sr, lane_off + (uint32_t)(c * 1024));
+    }
+    // the addend rows (empty resources read zeros): DEFER has the last source's only
+    u32x4 ad[ADD ? (DEFER ? 1 : S) : 1][ADD ? NCH : 1];
+    if constexpr (ADD) {
+#pragma unroll
+      for (int s = DEFER ? S - 1 : 0; s < S; ++s) {
+        const void* abase = P.dadd[s];
+        char* row = const_cast<char*>(
+            uniform_ptr(reinterpret_cast<uint64_t>(abase) + (uint64_t)t * ((uint64_t)P.dsrc_ld * 2)));
+        const __amdgpu_buffer_rsrc_t ar = row_rsrc(row, abase != nullptr ? row_size : 0u);
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) ad[DEFER ? 0 : s][c] = ld_row_nt(ar, lane_off + (uint32_t)(c * 1024));
+      }
+    }
+    const float glse = P.grad_lse != nullptr ? ld_scalar_f32(P.grad_lse + t) : 0.f;
+
+    // ---- sum(x^2), x.qw, x.G per source ----
+    float part[NP];
+#pragma unroll
+    for (int j = 0; j < NP; ++j) part[j] = 0.f;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const uint32_t xw = x[s][c][w];
+          part[s] = dot2_bf16(xw, xw, part[s]);
+          part[S + s] = __builtin_fmaf(bf_lo(xw), qw[c][2 * w], part[S + s]);
+          part[S + s] = __builtin_fmaf(bf_hi(xw), qw[c][2 * w + 1], part[S + s]);
+          part[2 * S + s] = dot2_bf16(xw, g[c][w], part[2 * S + s]);
+        }
+      }
+    }
+    // the wave's own LDS row: no barrier, only the order of its accesses
+    wave_reduce_to_lds<H2>(part, red[wave], lane);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+
+    // ---- softmax and the coefficients of dx, lane s per source ----
+    const int ls = lane % SEG;
+    const bool slot = ls < S;
+    const float t_ss = slot ? red[wave][ls] : 0.f;
+    const float t_dot = slot ? red[wave][S + ls] : 0.f;
+    const float t_gx = slot ? red[wave][2 * S + ls] : 0.f;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const float rl = __builtin_amdgcn_rsqf(t_ss * P.inv_d + P.eps);
+    const float ll = slot ? t_dot * rl : -__builtin_inff();
+    const float m = seg_max<SEG>(ll);
+    const float el = slot ? __expf(ll - m) : 0.f;
+    const float wl = el * (1.0f / seg_sum<SEG>(el));
+    const float go = seg_sum<SEG>(wl * t_gx);  // G . out = sum_s w_s (G . x_s)
+    // glse is added after G.x_s - G.out cancels (see route_bwd_body)
+    const float c1l = wl * (glse + (t_gx - go)) * rl;
+    const float c2l = -c1l * ll * rl * P.inv_d;
+    float c1[S], c2[S], wgt[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      wgt[s] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wl), s));
+      c1[s] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, c1l), s));
+      c2[s] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, c2l), s));
+    }
+    if constexpr (DEFER) {
+      // lanes >= S-1 fall outside the resource's range: their stores are dropped
+      char* crow = const_cast<char*>(uniform_ptr(reinterpret_cast<uint64_t>(P.coef) + (uint64_t)t * ((S - 1) * 16)));
+      st_row_nt(row_rsrc(crow, (uint32_t)((S - 1) * 16)), lane_off,
+                u32x4{as_u32(wl), as_u32(c1l), as_u32(c2l), 0u});
+    }
+
+    // ---- the gradient rows and the query gradient ----
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      // re-expanded from the packed words (opaque), not kept unpacked
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) asm volatile("" : "+v"(x[s][c]));
+      if (DEFER && s < S - 1) {
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            dq[c][2 * w] = __builtin_fmaf(c1[s], bf_lo(x[s][c][w]), dq[c][2 * w]);
+            dq[c][2 * w + 1] = __builtin_fmaf(c1[s], bf_hi(x[s][c][w]), dq[c][2 * w + 1]);
+          }
+        }
+        continue;
+      }
+      const __amdgpu_buffer_rsrc_t dr = row_at(P.dsrc[s], P.dsrc_ld, t);
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) {
+        u32x4 pk;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const uint32_t xw = x[s][c][w], gw = g[c][w];
+          const float x0 = bf_lo(xw), x1 = bf_hi(xw);
+          float d0 = __builtin_fmaf(c2[s], x0, __builtin_fmaf(c1[s], qw[c][2 * w], wgt[s] * bf_lo(gw)));
+          float d1 = __builtin_fmaf(c2[s], x1, __builtin_fmaf(c1[s], qw[c][2 * w + 1], wgt[s] * bf_hi(gw)));
+          dq[c][2 * w] = __builtin_fmaf(c1[s], x0, dq[c][2 * w]);
+          dq[c][2 * w + 1] = __builtin_fmaf(c1[s], x1, dq[c][2 * w + 1]);
+          if constexpr (ADD) {
+            d0 += bf_lo(ad[DEFER ? 0 : s][c][w]);
+            d1 += bf_hi(ad[DEFER ? 0 : s][c][w]);
+          }
+          pk[w] = pack_bf16(d0, d1);
+        }
+        st_row_nt(dr, lane_off + (uint32_t)(c * 1024), pk);
+      }
+    }
+  }
+
+  // ---- this workgroup's query-gradient partial: the waves' sums in a fixed order ----
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      dq_lds[wave * ROW4 + (c * 2 + h) * 64 + lane] =
+          make_float4(dq[c][4 * h], dq[c][4 * h + 1], dq[c][4 * h + 2], dq[c][4 * h + 3]);
+  }
+  __syncthreads();
+  float4* prow = reinterpret_cast<float4*>(P.dqw_part + (int64_t)blockIdx.x * P.d);
+  for (int j = tid; j < ROW4; j += 64 * ATTNRES_BWD_ROWS_WAVES) {
+    const int c = j >> 7, h = (j >> 6) & 1, l = j & 63;
+    if (c * 64 + l >= P.nchunk) continue;
+    float4 a = dq_lds[j];
+#pragma unroll
+    for (int w = 1; w < ATTNRES_BWD_ROWS_WAVES; ++w) {
+      const float4 b = dq_lds[w * ROW4 + j];
+      a.x += b.x;
+      a.y += b.y;
+      a.z += b.z;
+      a.w += b.w;
+    }
+    prow[(c * 64 + l) * 2 + h] = a;
+  }
 }
+
 
 // ------------------------------------------- segment of deferred sums --
 //
@@ -3738,7 +3960,7 @@ __device__ __forceinline__ void reduce_dqw_body(const attnres_reduce_params& P) 
   ROUTE_TYPES(S, 1) \
   ROUTE_TYPES(S, 2)
 
-// The build compiles this file once per module part (ATTNRES_PART = 0..10)
+// The build compiles this file once per module part (ATTNRES_PART = 0..11)
 // so the parts build in parallel; the host maps each symbol to its part.
 #ifndef ATTNRES_PART
 #define ATTNRES_PART 0
@@ -4052,12 +4274,42 @@ BWD_STREAM_ONE_DEFER(8, 6, 0)
 BWD_STREAM_ONE_DEFER(2, 8, 0) BWD_STREAM_ONE_DEFER(3, 8, 0) BWD_STREAM_ONE_DEFER(4, 8, 0)
 BWD_STREAM_ONE_DEFER(5, 8, 0) BWD_STREAM_ONE_DEFER(6, 8, 0) BWD_STREAM_ONE_DEFER(7, 8, 1)
 BWD_STREAM_ONE_DEFER(8, 8, 2) BWD_STREAM_ONE_DEFER(9, 8, 3)
-BWD_STREAM_ONE_DEFER(2, 2, 0) BWD_STREAM_ONE_DEFER(3, 2, 0) BWD_STREAM_ONE_DEFER(4, 2, 0)
-BWD_STREAM_ONE_DEFER(5, 2, 0) BWD_STREAM_ONE_DEFER(6, 2, 0) BWD_STREAM_ONE_DEFER(7, 2, 0)
-BWD_STREAM_ONE_DEFER(8, 2, 0)
-BWD_STREAM_ONE_DEFER(2, 1, 0) BWD_STREAM_ONE_DEFER(3, 1, 0) BWD_STREAM_ONE_DEFER(4, 1, 0)
-BWD_STREAM_ONE_DEFER(5, 1, 0) BWD_STREAM_ONE_DEFER(6, 1, 0) BWD_STREAM_ONE_DEFER(7, 1, 0)
-BWD_STREAM_ONE_DEFER(8, 1, 0)
+#endif
+
+// Row-per-wave backward of narrow rows: attnres_route_bwd_rows_c<NCH>_s<S>, with
+// addend rows (_add) and deferred block gradients (_defer).  Waves per SIMD by
+// the registers a token takes (S + 1 rows of 4 NCH, the query and its gradient
+// 16 NCH, and about 40).
+#define BWD_ROWS_EU(S, NCH, R) \
+  (4 * (NCH) * (R) + 16 * (NCH) + 40 <= 128 ? 4 : 4 * (NCH) * (R) + 16 * (NCH) + 40 <= 168 ? 3 : 2)
+#define BWD_ROWS_ONE(S, NCH)                                                                             \
+  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_BWD_ROWS_WAVES)                              \
+      __attribute__((amdgpu_waves_per_eu(BWD_ROWS_EU(S, NCH, (S) + 1))))                                 \
+      attnres_route_bwd_rows_c##NCH##_s##S(attnres_route_bwd_params P) {                                 \
+    route_bwd_rows_body<S, NCH>(P);                                                                      \
+  }
+#define BWD_ROWS_ADD(S, NCH)                                                                             \
+  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_BWD_ROWS_WAVES)                              \
+      __attribute__((amdgpu_waves_per_eu(BWD_ROWS_EU(S, NCH, 2 * (S) + 1))))                             \
+      attnres_route_bwd_rows_c##NCH##_s##S##_add(attnres_route_bwd_params P) {                           \
+    route_bwd_rows_body<S, NCH, true>(P);                                                                \
+  }
+#define BWD_ROWS_DEFER(S, NCH)                                                                           \
+  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_BWD_ROWS_WAVES)                              \
+      __attribute__((amdgpu_waves_per_eu(BWD_ROWS_EU(S, NCH, (S) + 2))))                                 \
+      attnres_route_bwd_rows_c##NCH##_s##S##_defer(attnres_route_bwd_params P) {                         \
+    route_bwd_rows_body<S, NCH, true, true>(P);                                                          \
+  }
+#define BWD_ROWS_S(S) \
+  BWD_ROWS_ONE(S, 1) BWD_ROWS_ONE(S, 2) BWD_ROWS_ONE(S, 3) BWD_ROWS_ADD(S, 1) BWD_ROWS_ADD(S, 2)
+#if ATTNRES_PART == 11 || defined(ATTNRES_ALL_PARTS)
+BWD_ROWS_S(1) BWD_ROWS_S(2) BWD_ROWS_S(3) BWD_ROWS_S(4) BWD_ROWS_S(5)
+BWD_ROWS_S(6) BWD_ROWS_S(7) BWD_ROWS_S(8) BWD_ROWS_S(9)
+BWD_ROWS_ADD(1, 3) BWD_ROWS_ADD(2, 3) BWD_ROWS_ADD(3, 3) BWD_ROWS_ADD(4, 3) BWD_ROWS_ADD(5, 3) BWD_ROWS_ADD(6, 3)
+BWD_ROWS_DEFER(2, 1) BWD_ROWS_DEFER(3, 1) BWD_ROWS_DEFER(4, 1) BWD_ROWS_DEFER(5, 1)
+BWD_ROWS_DEFER(6, 1) BWD_ROWS_DEFER(7, 1) BWD_ROWS_DEFER(8, 1)
+BWD_ROWS_DEFER(2, 2) BWD_ROWS_DEFER(3, 2) BWD_ROWS_DEFER(4, 2) BWD_ROWS_DEFER(5, 2)
+BWD_ROWS_DEFER(6, 2) BWD_ROWS_DEFER(7, 2) BWD_ROWS_DEFER(8, 2)
 #endif
 
 // Segments of deferred sums (the instances in ATTNRES_SEG_INSTANCES), a wave

@@ -1,0 +1,75 @@
+"""The row-per-wave kernels of narrow rows against the float64 oracle, at the
+row widths, source counts and row counts where they can go wrong: one chunk
+less and more than a whole KiB, the narrowest row, waves without a row."""
+
+import pytest
+import torch
+
+import kotodama_amd
+from kotodama_amd import _capi
+
+from .test_gpu_accumulate import _call, _case
+from .test_gpu_backward import Norm, _bwd_kernel_name, check_grad, make_case, oracle_grads
+
+pytestmark = pytest.mark.gpu
+
+
+def test_narrow_backward_policy(gpu):
+    auto = _capi.POLICY_AUTO
+    cus = torch.cuda.get_device_properties(gpu).multi_processor_count
+    assert _bwd_kernel_name(9, 4 * cus, 512, auto) == "attnres_route_bwd_rows_c1_s9"
+    assert _bwd_kernel_name(5, 8192, 520, auto) == "attnres_route_bwd_rows_c2_s5"
+    assert _bwd_kernel_name(5, 8192, 1536, auto) == "attnres_route_bwd_rows_c3_s5"
+    assert _bwd_kernel_name(5, 4 * cus - 1, 512, auto) == "attnres_route_bwd_bf_gbf_s5_v1"
+    assert _bwd_kernel_name(10, 8192, 512, auto) == "attnres_route_bwd_bf_gbf_s10_v1"
+    assert _bwd_kernel_name(5, 8192, 1544, auto) == "attnres_route_bwd_bf_gbf_s5_v1"
+
+
+CASES = [(8, 2, 3, None), (504, 9, 1030, None), (512, 9, 2049, None), (520, 1, 1025, None), (1000, 5, 1027, None),
+         (1024, 8, 1500, None), (1032, 3, 1100, torch.float32), (1536, 9, 1026, None), (1536, 4, 1, None)]
+
+
+@pytest.mark.parametrize("D,S,N,pd", CASES, ids=[f"D{c[0]}-S{c[1]}-N{c[2]}{'-pf32' if c[3] else ''}" for c in CASES])
+def test_narrow_backward_matches_oracle(gpu, D, S, N, pd):
+    print(f"narrow backward D={D} S={S} N={N} param={pd}", flush=True)
+    assert _bwd_kernel_name(S, N, D, _capi.POLICY_STREAM) == f"attnres_route_bwd_rows_c{(D + 511) // 512}_s{S}"
+    buf, query, gain, G = make_case(gpu, S, 0, 1, N, D, torch.bfloat16, seed=500 + S + D + N, param_dtype=pd)
+    buf.requires_grad_(True)
+    query.requires_grad_(True)
+    norm = Norm(gain.clone(), 1e-5)
+    mask = torch.ones(S, dtype=torch.bool, device=gpu)
+    prev = _capi.set_kernel_policy(_capi.POLICY_STREAM)
+    try:
+        out = kotodama_amd.route_static(buf, query, norm, mask, S)
+        (out.float() * G).sum().backward()
+        torch.cuda.synchronize()
+    finally:
+        _capi.set_kernel_policy(prev)
+    dx, dq, dg = oracle_grads(buf, S, query, norm.weight, G, 1e-5, pd or torch.bfloat16)
+    check_grad(buf.grad.reshape(S, -1, D), dx, torch.bfloat16, "dsources")
+    check_grad(query.grad, dq, query.dtype, "dquery")
+    check_grad(norm.weight.grad, dg, query.dtype, "dgain")
+
+
+@pytest.mark.parametrize("D,S,N", [(520, 9, 1030), (512, 1, 1025), (1536, 6, 1100)])
+def test_narrow_backward_adds_in_place(gpu, D, S, N):
+    # addend rows (here the gradient rows themselves) for every other source: those sources get
+    # the plain gradient plus the addend within one rounding of it, the others its exact bits
+    src, q, gain, gout, addend = _case(gpu, S, N, D, torch.bfloat16, 900 + S)
+    prev = _capi.set_kernel_policy(_capi.POLICY_STREAM)
+    try:
+        plain = torch.full_like(src, 3.0)
+        dq0, dg0 = _call(gpu, src, q, gain, gout, plain, None)
+        grads = addend.clone()
+        dq1, dg1 = _call(gpu, src, q, gain, gout, grads, [grads[s] if s % 2 == 0 else None for s in range(S)])
+    finally:
+        _capi.set_kernel_policy(prev)
+    assert torch.equal(dq0, dq1) and torch.equal(dg0, dg1)
+    for s in range(S):
+        if s % 2:
+            assert torch.equal(grads[s], plain[s])
+        else:
+            # plain is rounded to bf16 (2^-9 of it) and the sum once more (2^-9 of the sum)
+            want = plain[s].double() + addend[s].double()
+            bar = 2.0**-8 * (plain[s].double().abs() + want.abs()) + 1e-30
+            assert ((grads[s].double() - want).abs() <= bar).all()
