@@ -11,6 +11,9 @@ Steps (all outputs under ``kotodama_amd/lib/``):
    shared library, linked against ROCm's ``libamdhip64.so.7``.  Loaded after ``import torch``,
    the dynamic linker binds that soname to the HIP runtime torch already
    loaded, so streams and device memory are shared with torch.
+5. ``g++`` compiles ``csrc/attnres_torch.cpp`` against torch's headers into
+   ``_attnres_torch.so``, the CPython extension through which the eager torch
+   layer calls that library.
 
 Run ``python -m kotodama_amd.build`` or call :func:`build`.
 """
@@ -28,6 +31,7 @@ CSRC = PKG / "csrc"
 LIBDIR = PKG / "lib"
 INCLUDE = PKG.parent / "include"
 LIB_NAME = "libattnres_hip.so"
+NATIVE_NAME = "_attnres_torch.so"
 ROCM = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
 ARCH = "gfx950"
 NUM_PARTS = 12
@@ -44,6 +48,17 @@ HIP_FLAGS = [
     "-Xclang",
     "-packed-fp32-ops",
 ]
+
+
+def _native_cmd(out: Path) -> list[str]:
+    """Compile the torch layer's extension to an object file (the link follows the C-ABI library's)."""
+    import sysconfig
+
+    from torch.utils.cpp_extension import include_paths
+
+    incs = [f"-isystem{p}" for p in [*include_paths(), ROCM / "include", sysconfig.get_paths()["include"]]]
+    return ["g++", "-c", "-fPIC", "-O2", "-std=c++17", "-Wall", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__",
+            "-DUSE_ROCM", f"-I{INCLUDE}", *incs, str(CSRC / "attnres_torch.cpp"), "-o", str(out)]
 
 
 def _run(cmd: list[str], cwd: Path | None = None) -> None:
@@ -64,7 +79,9 @@ def build(verbose: bool = False, out_dir: Path | None = None, defines: tuple = (
     extra = [f"-D{d}" for d in defines]
     with tempfile.TemporaryDirectory(prefix="attnres_build_", dir=libdir) as tmp:
         tmpd = Path(tmp)
-        procs = []
+        native_o = tmpd / "attnres_torch.o"
+        native = _native_cmd(native_o)
+        procs = [(native, subprocess.Popen(native, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True))]
         for part in range(NUM_PARTS):
             out = tmpd / f"attnres_gfx950_part{part}.hsaco"
             cmd = [hipcc, *HIP_FLAGS, *extra, f"-DATTNRES_PART={part}", f"-I{CSRC}", str(CSRC / "attnres_kernels.hip"),
@@ -75,7 +92,7 @@ def build(verbose: bool = False, out_dir: Path | None = None, defines: tuple = (
         for cmd, p in procs:
             so, se = p.communicate()
             if p.returncode != 0:
-                raise RuntimeError(f"hipcc failed ({p.returncode}): {' '.join(cmd)}\n{so}\n{se}")
+                raise RuntimeError(f"{Path(cmd[0]).name} failed ({p.returncode}): {' '.join(cmd)}\n{so}\n{se}")
         blob_o = tmpd / "attnres_blob.o"
         _run(["gcc", "-c", f"-I{tmpd}", str(CSRC / "attnres_blob.S"), "-o", str(blob_o)])
         noalloc_o = tmpd / "attnres_noalloc.o"
@@ -108,8 +125,16 @@ def build(verbose: bool = False, out_dir: Path | None = None, defines: tuple = (
                 str(so_tmp),
             ]
         )
+        import torch
+
+        torch_lib = Path(torch.__file__).parent / "lib"
+        native_tmp = tmpd / NATIVE_NAME
+        _run(["g++", "-shared", str(native_o), f"-L{tmpd}", "-lattnres_hip", f"-L{torch_lib}", "-ltorch_python",
+              "-ltorch_cpu", "-ltorch_hip", "-lc10_hip", "-lc10", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{torch_lib}",
+              "-o", str(native_tmp)])
         final = libdir / LIB_NAME
         os.replace(so_tmp, final)  # atomic: a reader never sees a half-written library
+        os.replace(native_tmp, libdir / NATIVE_NAME)
     if verbose:
         print(f"built {final}", flush=True)
     return final

@@ -42,6 +42,7 @@ import torch
 from torch import Tensor
 
 from . import _capi
+from ._native import native
 
 _DTYPE_CODES = {torch.float32: _capi.DTYPE_F32, torch.bfloat16: _capi.DTYPE_BF16}
 _CODE_DTYPES = {v: k for k, v in _DTYPE_CODES.items()}
@@ -589,6 +590,28 @@ def _route_backward(ctx, g_out, g_w, g_lse, g_inv, g_logits):
 
 route.register_autograd(_route_backward, setup_context=_route_setup_context)
 
+# How the native calls hand back a routing result (attnres_torch.cpp): the rows
+# alone, the five outputs with None or with empty tensors where not requested.
+_ROWS, _TUPLE, _PLACEHOLDERS = 1, 2, 3
+
+
+class _EagerRoute(type(route)):
+    """``route`` as the registered op whose plain eager calls, recorded by
+    autograd or not, take the native path: the same outputs and gradients
+    without the dispatcher's Python.  Traced, transformed and watched calls
+    (and those the native path leaves alone) go to the op."""
+
+    def __call__(self, buf, num_sources, query, gain, eps, out_dtype, want_weights, want_aux):
+        if not torch.compiler.is_compiling() and isinstance(buf, Tensor):
+            res = native.route(buf, num_sources, query, gain, eps, out_dtype, want_weights, want_weights, want_aux,
+                               _PLACEHOLDERS, not _inactive_grads_discarded(buf, num_sources))
+            if res is not None:
+                return res
+        return super().__call__(buf, num_sources, query, gain, eps, out_dtype, want_weights, want_aux)
+
+
+route.__class__ = _EagerRoute
+
 
 def _route_list_setup_context(ctx, inputs, output):
     sources, query, gain, eps, out_dtype, _, _ = inputs
@@ -623,6 +646,21 @@ def _route_list_backward(ctx, g_out, g_w, g_lse, g_inv, g_logits):
 
 
 route_list.register_autograd(_route_list_backward, setup_context=_route_list_setup_context)
+
+
+class _EagerRouteList(type(route_list)):
+    """``route_list``, its plain eager calls native as ``route``'s."""
+
+    def __call__(self, sources, query, gain, eps, out_dtype, want_weights, want_aux):
+        if not torch.compiler.is_compiling():
+            res = native.route_list(sources, query, gain, eps, out_dtype, want_weights, want_weights, want_aux,
+                                    _PLACEHOLDERS, True)
+            if res is not None:
+                return res
+        return super().__call__(sources, query, gain, eps, out_dtype, want_weights, want_aux)
+
+
+route_list.__class__ = _EagerRouteList
 
 
 # ------------------------------------------------- summed block gradients --
@@ -741,6 +779,14 @@ class GradSegments:
         nb = k + 1
         part_in = [self.part.get(j) for j in range(nb)]
         csum_in = [self.csum.get(j) for j in range(nb)]
+        res = native.gather_seg(terms, part_in, csum_in, x, addend)
+        if res is not None:
+            out, parts, csums = res
+            for j in range(k):
+                self.part[j], self.csum[j] = parts[j], csums[j]
+            self.part.pop(k, None)
+            self.csum.pop(k, None)
+            return out
         part_out = [p if p is not None else torch.empty((n_tok, d), device=x.device, dtype=x.dtype)
                     for p in part_in[:k]]
         csum_out = [c if c is not None else torch.empty(n_tok, device=x.device, dtype=torch.float32)
@@ -844,12 +890,18 @@ def commit_block(block: Tensor, slot: GradSlot) -> Tensor:
 
 
 def _route_rows_forward(sources, query, gain, eps, out_dtype) -> Tensor:
+    res = native.route_list(sources, query, gain, eps, out_dtype, False, False, False, _ROWS, False)
+    if res is not None:
+        return res
     out = _route_list_impl(list(sources), query, gain, eps, out_dtype, False, False, placeholders=False)[0]
     return out.view(out.shape[1:])
 
 
 def _route_rows_backward(sources, grads, adds, query, gain, eps, grad_out) -> tuple[Tensor, Optional[Tensor]]:
     """attnres_route_bwd(_add) into ``grads``; ``adds[s]`` is None or the row block added to source s's gradient."""
+    res = native.bwd_rows(sources, grads, adds, query, gain, eps, grad_out)
+    if res is not None:
+        return res
     device = sources[0].device
     d = sources[0].shape[-1]
     n = sources[0].numel() // d
@@ -863,6 +915,9 @@ def _route_rows_backward_defer(sources, query, gain, eps, grad_out, grad_add):
     """attnres_route_bwd_defer: (partial's gradient, (n, S-1, 4) coefficient
     records, folded query, grad_out as (n, D) rows, grad_query, grad_gain),
     or None when the library has no deferred kernel for the call."""
+    res = native.bwd_defer(sources, query, gain, eps, grad_out, grad_add)
+    if res is not None:
+        return res
     p = sources[-1]
     device = p.device
     d = p.shape[-1]
@@ -893,6 +948,9 @@ def _route_rows_backward_defer(sources, query, gain, eps, grad_out, grad_add):
 
 def _route_rows_step(committed, partial, delta, query, gain, eps, out_dtype) -> tuple[Tensor, Tensor]:
     """attnres_route_step: (routed rows, partial + delta in a new tensor)."""
+    res = native.step(committed, partial, delta, query, gain, eps, out_dtype)
+    if res is not None:
+        return res
     device = _require_device(*committed, partial, delta, query, gain)
     ref = partial
     for t in (*committed, delta):
@@ -1087,13 +1145,13 @@ def _merge_fake(partial, query, inter, inter_lse, eps):
 
 # ------------------------------------------------------------ eager calls --
 #
-# Called through the dispatcher, each op costs ~24 us of host time per call
-# (measured on an MI355X host: the dispatcher, four placeholder outputs, the ctypes call),
-# several times the kernel of a small routing call.  The drop-ins go through
-# the helpers below, which launch the same implementation directly when there
-# is nothing to record: eager mode, no autograd graph to build, no tracing,
-# no dispatch or function mode, plain tensors.  Otherwise they call the op.
-# Outputs that were not requested are None on the direct path.
+# Through the dispatcher one call costs ~24 us of host time (the dispatcher,
+# four placeholder outputs, the ctypes call), several times the kernel of a
+# small routing call.  The drop-ins go through the helpers below.  A plain
+# call (eager, no tracing, no dispatch or function mode, plain contiguous
+# tensors) is launched by the native extension; what that leaves alone is
+# launched here directly when there is nothing to record, and goes to the op
+# otherwise.  Outputs that were not requested are None on the direct paths.
 
 _PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
 
@@ -1121,16 +1179,55 @@ def route_call(buf, num_sources, query, gain, eps, out_dtype, want_weights=False
 
     ``want_lse`` asks for the lse without the weights (the op ties them).
     """
+    lse = want_weights if want_lse is None else want_lse
+    if not torch.compiler.is_compiling():
+        res = native.route(buf, num_sources, query, gain, eps, out_dtype, want_weights, lse, want_aux, _TUPLE, None)
+        if res is not None:
+            return res
+        if lse and not want_weights and isinstance(buf, Tensor):
+            # recorded by autograd: the op would also store the weights
+            res = native.route(buf, num_sources, query, gain, eps, out_dtype, False, True, want_aux, _TUPLE,
+                               not _inactive_grads_discarded(buf, num_sources))
+            if res is not None:
+                return res
     if _eager_direct(buf, query, gain):
         return _route_impl(buf, num_sources, query, gain, eps, out_dtype, want_weights, want_aux, placeholders=False,
                            want_lse=want_lse)
     return route(buf, num_sources, query, gain, eps, out_dtype, want_weights or bool(want_lse), want_aux)
 
 
+def route_rows(buf, num_sources, query, gain, eps) -> Tensor:
+    """The routed rows of a stacked buffer in the einsum branch's dtype, without the query dimension."""
+    if not torch.compiler.is_compiling():
+        out = native.route(buf, num_sources, query, gain, eps, None, False, False, False, _ROWS, None)
+        if out is not None:
+            return out
+    return route_call(buf, num_sources, query, gain, eps, _promoted(buf, query, gain))[0].squeeze(0)
+
+
+def route_list_rows(sources, query, gain, eps) -> Tensor:
+    """:func:`route_rows` over a list of separate blocks."""
+    if not torch.compiler.is_compiling():
+        out = native.route_list(sources, query, gain, eps, None, False, False, False, _ROWS, False)
+        if out is not None:
+            return out
+    return route_list_call(sources, query, gain, eps, _promoted(sources[0], query, gain))[0].squeeze(0)
+
+
+def _promoted(src: Tensor, query: Tensor, gain: Tensor) -> torch.dtype:
+    return torch.promote_types(src.dtype, torch.promote_types(query.dtype, gain.dtype))
+
+
 def route_list_call(sources, query, gain, eps, out_dtype, want_weights=False, want_aux=False,
                     want_lse=None) -> tuple:
     """:func:`route_list`, launched directly when nothing needs the dispatcher (``want_lse`` as in
     :func:`route_call`)."""
+    lse = want_weights if want_lse is None else want_lse
+    if not torch.compiler.is_compiling():
+        res = native.route_list(sources, query, gain, eps, out_dtype, want_weights, lse, want_aux, _TUPLE,
+                                bool(lse and not want_weights))
+        if res is not None:
+            return res
     if _eager_direct(query, gain, *sources):
         return _route_list_impl(sources, query, gain, eps, out_dtype, want_weights, want_aux, placeholders=False,
                                 want_lse=want_lse)
@@ -1139,6 +1236,10 @@ def route_list_call(sources, query, gain, eps, out_dtype, want_weights=False, wa
 
 def merge_call(partial, query, inter, inter_lse, eps) -> Tensor:
     """The merged rows of :func:`merge`, launched directly when nothing needs the dispatcher."""
+    if not torch.compiler.is_compiling():
+        out = native.merge(partial, query, inter, inter_lse, eps)
+        if out is not None:
+            return out
     if _eager_direct(partial, query, inter, inter_lse):
         return _merge_impl(partial, query, inter, inter_lse, eps, aux=False)[0]
     return merge(partial, query, inter, inter_lse, eps)[0]
@@ -1292,6 +1393,10 @@ def block_step(
 
 def block_step_call(arena, n_committed, commit, delta, query, gain, eps, want_weights=False) -> tuple:
     """:func:`block_step`, launched directly when nothing needs the dispatcher."""
+    if not torch.compiler.is_compiling():
+        res = native.block_step(arena, n_committed, commit, delta, query, gain, eps, want_weights)
+        if res is not None:
+            return res
     if _eager_direct(arena, delta, query, gain):
         return _block_step_impl(arena, n_committed, commit, delta, query, gain, eps, want_weights, placeholders=False)
     return block_step(arena, n_committed, commit, delta, query, gain, eps, want_weights)

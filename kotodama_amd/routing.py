@@ -46,11 +46,9 @@ def route_static(
     of active slots is routed by passing their pointers.
     """
     gain = norm.weight
-    out_dtype = _out_dtype(buf.dtype, query, gain)
     if num_active:
-        n = int(num_active)
-        res = ops.route_call(buf, n, query, gain, float(norm.eps), out_dtype)
-        return res[0].squeeze(0)
+        return ops.route_rows(buf, int(num_active), query, gain, float(norm.eps))
+    out_dtype = _out_dtype(buf.dtype, query, gain)
     idx = [i for i, a in enumerate(active_mask.reshape(-1).tolist()) if a]
     if idx == list(range(len(idx))):
         res = ops.route_call(buf, len(idx), query, gain, float(norm.eps), out_dtype)
@@ -66,10 +64,7 @@ def block_attn_res_from_list(sources: Sequence[Tensor], query: Tensor, norm) -> 
     -inf; the padded slots get weight exactly 0, so routing over the list
     itself gives the same result without building the padded buffer.
     """
-    gain = norm.weight
-    out_dtype = _out_dtype(sources[0].dtype, query, gain)
-    res = ops.route_list_call(list(sources), query, gain, float(norm.eps), out_dtype)
-    return res[0].squeeze(0)
+    return ops.route_list_rows(list(sources), query, norm.weight, float(norm.eps))
 
 
 def route_weights(buf: Tensor, num_active: int, query: Tensor, norm) -> tuple[Tensor, Tensor, Tensor]:
