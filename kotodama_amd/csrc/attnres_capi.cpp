@@ -746,6 +746,15 @@ void kernel_name_of(const RouteChoice& ch, int num_sources, int num_queries, boo
   }
 }
 
+// Source bytes up to which the row-per-workgroup kernels read the sources
+// without the non-temporal hint: what fits the eight 4 MiB L2s beside the
+// sublayer output and the routed rows.  Consecutive routing points read the
+// same blocks: 65 decode points of 256 rows (hidden 4096, up to 19 MB of
+// sources) 359 -> 322 us, 57 points of 1501 rows (hidden 1024) 362 -> 328.
+// Over larger sources the hint is better: hidden 768, S = 5, 32768 rows
+// 54.1 us with it and 59.2 without, at 8192 rows (63 MB) 14.4 and 15.4.
+constexpr int64_t kCachedSourceBytes = 24 << 20;
+
 // Shared validation + launch of the route kernel.  `mode`/`delta` are the
 // fused partial-update inputs of attnres_block_step.
 // The kernel choice of one merge call, shared by the launch and the name
@@ -899,6 +908,7 @@ int route_launch(const void* const* sources, int num_sources, int64_t num_tokens
   P.num_sources = num_sources;
   P.block = block;
   P.out_batch = out_batch;
+  P.src_cached = num_sources * num_tokens * (int64_t)hidden * esize(src_dtype) <= kCachedSourceBytes;
   P.eps = eps;
   P.inv_d = 1.0f / (float)hidden;
   // The streaming kernels run one 4-wave workgroup per CU from 6 KiB rows: at

@@ -173,6 +173,14 @@ __device__ __forceinline__ T ldg_global(const char* p) {
   return *g;
 #endif
 }
+// The same with or without the hint: data that other workgroups or the next
+// call read again stays in the caches.
+template <bool NT, typename T>
+__device__ __forceinline__ T ldg_hint(const char* p) {
+  const __attribute__((address_space(1))) T* g = (const __attribute__((address_space(1))) T*)(p);
+  if constexpr (NT) return __builtin_nontemporal_load(g);
+  else return *g;
+}
 template <typename T>
 __device__ __forceinline__ void stg(void* p, T v) {
   *reinterpret_cast<T*>(p) = v;
@@ -351,8 +359,10 @@ __device__ __forceinline__ void load_qw(const attnres_route_params& P, int q, in
 }
 
 // A parameter chunk (VEC elements, bf16 or fp32 by a runtime flag) loaded
-// packed; converted with param_elem after every load of the prologue has been
-// issued, so the loads share one wait.
+// packed, without the non-temporal hint: every workgroup reads the same
+// parameters (with it, 65 decode points of 256 rows took 399 us instead of
+// 354, 57 points of 1501 rows 396 instead of 351).  Converted with param_elem
+// after every load of the prologue has been issued, so the loads share one wait.
 template <int VEC>
 struct ParamRaw {
   u32x4 w[VEC == 8 ? 2 : 1];
@@ -362,15 +372,15 @@ __device__ __forceinline__ void load_param_raw(const void* base, int chunk, bool
   const char* b = reinterpret_cast<const char*>(base);
   if (bf16) {
     if constexpr (VEC == 8) {
-      r.w[0] = ldg_global<u32x4>(b + (int64_t)chunk * 16);
+      r.w[0] = ldg_hint<false, u32x4>(b + (int64_t)chunk * 16);
       r.w[1] = u32x4{0, 0, 0, 0};
     } else {
-      const u32x2 t = ldg_global<u32x2>(b + (int64_t)chunk * 8);
+      const u32x2 t = ldg_hint<false, u32x2>(b + (int64_t)chunk * 8);
       r.w[0] = u32x4{t[0], t[1], 0, 0};
     }
   } else {
 #pragma unroll
-    for (int h = 0; h < VEC / 4; ++h) r.w[h] = ldg_global<u32x4>(b + ((int64_t)chunk * VEC + 4 * h) * 4);
+    for (int h = 0; h < VEC / 4; ++h) r.w[h] = ldg_hint<false, u32x4>(b + ((int64_t)chunk * VEC + 4 * h) * 4);
   }
 }
 template <int VEC>
@@ -520,7 +530,8 @@ __device__ __forceinline__ void route_body(const attnres_route_params& P) {
   constexpr int SX = S > 0 ? S : 1;
   u32x4 x[SX][V];
   u32x4 dvr[V];
-  auto load_row = [&](int64_t t) {
+  auto load_row_as = [&](int64_t t, auto stream) {
+    constexpr bool NT = decltype(stream)::value;
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       const char* row = reinterpret_cast<const char*>(P.src[s]) + t * row_bytes_ld;
@@ -529,15 +540,21 @@ __device__ __forceinline__ void route_body(const attnres_route_params& P) {
         if (s == S - 1 && P.mode == ATTNRES_MODE_SET) {
           x[s][k] = u32x4{0, 0, 0, 0};
         } else {
-          x[s][k] = ok[k] ? ldg_global<u32x4>(row + (int64_t)chunk[k] * 16) : u32x4{0, 0, 0, 0};
+          x[s][k] = ok[k] ? ldg_hint<NT, u32x4>(row + (int64_t)chunk[k] * 16) : u32x4{0, 0, 0, 0};
         }
       }
     }
     if (S > 0 && P.mode != ATTNRES_MODE_PLAIN) {
       const char* drow = reinterpret_cast<const char*>(P.delta) + t * P.delta_ld * C::BYTES;
 #pragma unroll
-      for (int k = 0; k < V; ++k) dvr[k] = ok[k] ? ldg_global<u32x4>(drow + (int64_t)chunk[k] * 16) : u32x4{0, 0, 0, 0};
+      for (int k = 0; k < V; ++k) dvr[k] = ok[k] ? ldg_hint<NT, u32x4>(drow + (int64_t)chunk[k] * 16) : u32x4{0, 0, 0, 0};
     }
+  };
+  // Source rows small enough to stay in the L2s (P.src_cached) are read without
+  // the non-temporal hint: the next routing point reads the same blocks.
+  auto load_row = [&](int64_t t) {
+    if (P.src_cached) load_row_as(t, std::false_type{});
+    else load_row_as(t, std::true_type{});
   };
   if (S > 0 && (int64_t)blockIdx.x < P.n_tokens) load_row(blockIdx.x);
   if constexpr (!MULTIQ) {

@@ -64,6 +64,7 @@ typedef struct attnres_route_params {
                            dispatch packet, so it costs no vector load) */
   int32_t out_batch;    /* streaming kernels: finished output rows each wave stages in
                            (dynamic) LDS and stores together; 1 = store each row at once */
+  int32_t src_cached;   /* row-per-workgroup kernels: read the sources without the non-temporal hint */
   float eps;
   float inv_d;
 } attnres_route_params;
