@@ -112,8 +112,10 @@ struct DeviceState {
   KernelSlot bwd_rows[3 * 3 * 10];  // narrow rows' backward: plain / _add / _defer x row KiB (1..3) x S (1..9)
   KernelSlot reduce_stage, reduce_cols, reduce_fin;
   KernelSlot merge_bwd[kMergeFuncs];
+  KernelSlot merge_bwd_rows[6];  // its row-per-wave form: row KiB (1..6)
   KernelSlot bwd_mq[kBwdFuncs];  // batched-query backward: (source, grad_out) dtypes x S x V
   KernelSlot bwd_dqw[4];         // source dtype x V
+  KernelSlot bwd_mqg_rows[2 * 2 * 9];  // its row-per-wave form: chunks per lane x query groups x S
   KernelSlot bwd_mqg[2 * 9];     // batched-query backward on the matrix cores: query groups x S
   KernelSlot bwd_defer[2 * 10];  // row-per-wave backward with deferred block gradients: 6 / 8 KiB rows x S
   KernelSlot gather_seg[4 * ATTNRES_SEG_MAX_BLOCKS];  // segment sums: row width x blocks
@@ -447,8 +449,8 @@ int get_bwd_rows(DeviceState& st, int nch, int s, BwdRowsVariant var, hipFunctio
                   64 * ATTNRES_BWD_ROWS_WAVES, 0, f, bpc);
 }
 // Its grid: two workgroups per CU where they fit (measured in the kernel's comment).
-int bwd_rows_grid(int64_t num_tokens, int num_cus, int bpc) {
-  const int limit = tuning().bwd_per_cu > 0 ? tuning().bwd_per_cu : 2;
+int bwd_rows_grid(int64_t num_tokens, int num_cus, int bpc, int per_cu = 2) {
+  const int limit = tuning().bwd_per_cu > 0 ? tuning().bwd_per_cu : per_cu;
   const int64_t need = (num_tokens + ATTNRES_BWD_ROWS_WAVES - 1) / ATTNRES_BWD_ROWS_WAVES;
   const int64_t cap = (int64_t)num_cus * (bpc < limit ? bpc : limit);
   return (int)(need < cap ? need : cap);
@@ -551,11 +553,39 @@ int get_bwd_mqg(DeviceState& st, int s, int nq4, int block, size_t lds, hipFunct
   return slot_get(st, st.bwd_mqg[(nq4 - 1) * 9 + s], kBwdMqgPart, name, block, lds, f, bpc);
 }
 
+// Its row-per-wave form for rows of at most 128 chunks (four rows per
+// workgroup): chunks per lane, or 0 for wider rows.  Faster at every S and row
+// count measured (1000 to 32768 rows: 4-21% of the whole backward), at the
+// occupancy limit as the row-per-workgroup form (two per CU 0-7% slower).
+int mqg_rows_v(int nchunk) { return nchunk <= 64 ? 1 : nchunk <= 128 ? 2 : 0; }
+int get_bwd_mqg_rows(DeviceState& st, int v, int s, int nq4, size_t lds, hipFunction_t* f, int* bpc) {
+  char name[96];
+  snprintf(name, sizeof(name), "attnres_route_bwd_mqg_rows_v%d_s%d_q%d", v, s, nq4);
+  return slot_get(st, st.bwd_mqg_rows[((v - 1) * 2 + nq4 - 1) * 9 + s], kBwdMqgPart, name,
+                  64 * ATTNRES_BWD_ROWS_WAVES, lds, f, bpc);
+}
+
 int get_merge_bwd(DeviceState& st, bool pbf, bool ibf, int v, int block, hipFunction_t* f, int* bpc) {
   char name[96];
   snprintf(name, sizeof(name), "attnres_merge_bwd_%s_%s_v%d", pbf ? "bf" : "f32", ibf ? "bf" : "f32", v);
   return slot_get(st, st.merge_bwd[((pbf ? 0 : 2) + (ibf ? 0 : 1)) * 2 + (v - 1)], kReducePart, name, block, 0, f,
                   bpc);
+}
+
+int get_merge_bwd_rows(DeviceState& st, int nch, hipFunction_t* f, int* bpc) {
+  char name[96];
+  snprintf(name, sizeof(name), "attnres_merge_bwd_rows_c%d", nch);
+  return slot_get(st, st.merge_bwd_rows[nch - 1], kBwdRowsPart, name, 64 * ATTNRES_BWD_ROWS_WAVES, 0, f, bpc);
+}
+// Row KiB (rounded up) of the merge backward's row-per-wave kernel (bf16 rows of
+// up to 6 KiB) for this call, or 0 for the row-per-workgroup one.  AUTO takes
+// it from two rows per CU: at 512 rows it measured 1-10% faster at every width,
+// at 300 rows even to 3% slower and at 64 rows of 5-6 KiB 6-10% slower.
+int merge_bwd_rows_nch(bool pbf, bool ibf, int hidden, int64_t num_tokens, int num_cus) {
+  if (!pbf || !ibf || hidden > 3072 || num_tokens >= (int64_t)1 << 31) return 0;
+  const int policy = g_policy.load(std::memory_order_relaxed);
+  const int want = policy == ATTNRES_POLICY_STREAM ? 1 : policy == ATTNRES_POLICY_WORKGROUP ? 0 : tuning().stream;
+  return want == 1 || (want < 0 && num_tokens >= 2LL * num_cus) ? (hidden + 511) / 512 : 0;
 }
 
 int get_reduce(DeviceState& st, ReduceFns* out) {
@@ -1076,7 +1106,11 @@ int attnres_route_bwd_queries_kernel_name(int num_sources, int hidden, int src_d
   const size_t lds = mqg_lds_bytes(num_queries, nchunk);
   if (bwd_mqg_shape(bf, gbf, param_dtype == ATTNRES_DTYPE_BF16, num_sources, num_queries, nchunk) &&
       lds + kMqgStaticLds <= (size_t)st->max_lds) {
-    snprintf(buf, (size_t)buf_len, "attnres_route_bwd_mqg_s%d_q%d", num_sources, (num_queries + 3) / 4);
+    const int rv = mqg_rows_v(nchunk);
+    if (rv > 0)
+      snprintf(buf, (size_t)buf_len, "attnres_route_bwd_mqg_rows_v%d_s%d_q%d", rv, num_sources, (num_queries + 3) / 4);
+    else
+      snprintf(buf, (size_t)buf_len, "attnres_route_bwd_mqg_s%d_q%d", num_sources, (num_queries + 3) / 4);
   } else if (bwd_mq_available(bf, num_sources, v)) {
     snprintf(buf, (size_t)buf_len, "attnres_route_bwd_mq_%s_g%s_s%d_v%d", bf ? "bf" : "f32", gbf ? "bf" : "f32",
              num_sources, v);
@@ -1758,10 +1792,13 @@ int attnres_route_bwd_queries(const void* const* sources, int num_sources, int64
                 "is not built for %d chunks per thread; call attnres_route_bwd once per query",
                 num_sources, mqg_lds, v);
   const int block = v == 1 ? round64(nchunk) : round64((nchunk + 1) / 2);
-  const int mqg_block = round64((nchunk + 1) / 2);
+  const int rows_v = mqg ? mqg_rows_v(nchunk) : 0;
+  const int mqg_block = rows_v > 0 ? 64 * ATTNRES_BWD_ROWS_WAVES : round64((nchunk + 1) / 2);
   hipFunction_t f = nullptr, fq = nullptr;
   int bpc = 1, bpcq = 1;
-  if (mqg) {
+  if (rows_v > 0) {
+    rc = get_bwd_mqg_rows(*st, rows_v, num_sources, (num_queries + 3) / 4, mqg_lds, &f, &bpc);
+  } else if (mqg) {
     rc = get_bwd_mqg(*st, num_sources, (num_queries + 3) / 4, mqg_block, mqg_lds, &f, &bpc);
   } else {
     rc = get_bwd_mq(*st, bf, grad_out_dtype == ATTNRES_DTYPE_BF16, num_sources, v, block, &f, &bpc);
@@ -1817,7 +1854,8 @@ int attnres_route_bwd_queries(const void* const* sources, int num_sources, int64
   int per_cu = mqg ? bpc : (bpc < 2 ? bpc : 2);
   if (tuning().bwd_per_cu > 0 && tuning().bwd_per_cu < per_cu) per_cu = tuning().bwd_per_cu;
   int64_t grid = (int64_t)st->num_cus * per_cu;
-  if (grid > num_tokens) grid = num_tokens;
+  const int64_t units = rows_v > 0 ? (num_tokens + ATTNRES_BWD_ROWS_WAVES - 1) / ATTNRES_BWD_ROWS_WAVES : num_tokens;
+  if (grid > units) grid = units;
   rc = mqg ? launch(f, (int)grid, mqg_block, P, stream, 1, mqg_lds) : launch(f, (int)grid, block, P, stream);
   if (rc != ATTNRES_OK || !want_q) return rc;
 
@@ -1873,18 +1911,27 @@ int attnres_merge_bwd(const void* partial, int64_t num_tokens, int hidden, int p
   DeviceState* st = nullptr;
   int rc = ensure_loaded(&st);
   if (rc != ATTNRES_OK) return rc;
-  // two chunks per thread where that leaves at least two waves per row
-  // (measured 5% faster at D = 3072 than one chunk per thread)
-  int v = round64(nchunk) > kMaxThreads || round64((nchunk + 1) / 2) >= 128 ? 2 : 1;
-  if (tuning().force_v == 1 && round64(nchunk) <= kMaxThreads) v = 1;  // measurement knob (ATTNRES_V)
-  const int block = v == 1 ? round64(nchunk) : round64((nchunk + 1) / 2);
   hipFunction_t f = nullptr;
-  int bpc = 1;
-  rc = get_merge_bwd(*st, pbf, ibf, v, block, &f, &bpc);
-  if (tuning().bwd_per_cu > 0 && tuning().bwd_per_cu < bpc) bpc = tuning().bwd_per_cu;
-  if (rc != ATTNRES_OK) return rc;
-  int64_t grid = (int64_t)st->num_cus * (bpc < kBwdMaxPerCu ? bpc : kBwdMaxPerCu);
-  if (grid > num_tokens) grid = num_tokens;
+  int bpc = 1, block = 0;
+  int64_t grid = 0;
+  const int rnch = merge_bwd_rows_nch(pbf, ibf, hidden, num_tokens, st->num_cus);
+  if (rnch > 0) {
+    block = 64 * ATTNRES_BWD_ROWS_WAVES;
+    rc = get_merge_bwd_rows(*st, rnch, &f, &bpc);
+    if (rc != ATTNRES_OK) return rc;
+    grid = bwd_rows_grid(num_tokens, st->num_cus, bpc, rnch <= 4 ? 2 : 1);
+  } else {
+    // two chunks per thread where that leaves at least two waves per row
+    // (measured 5% faster at D = 3072 than one chunk per thread)
+    int v = round64(nchunk) > kMaxThreads || round64((nchunk + 1) / 2) >= 128 ? 2 : 1;
+    if (tuning().force_v == 1 && round64(nchunk) <= kMaxThreads) v = 1;  // measurement knob (ATTNRES_V)
+    block = v == 1 ? round64(nchunk) : round64((nchunk + 1) / 2);
+    rc = get_merge_bwd(*st, pbf, ibf, v, block, &f, &bpc);
+    if (rc != ATTNRES_OK) return rc;
+    if (tuning().bwd_per_cu > 0 && tuning().bwd_per_cu < bpc) bpc = tuning().bwd_per_cu;
+    grid = (int64_t)st->num_cus * (bpc < kBwdMaxPerCu ? bpc : kBwdMaxPerCu);
+    if (grid > num_tokens) grid = num_tokens;
+  }
   const int64_t need = grid * (int64_t)hidden * (int64_t)sizeof(float);
   if (workspace == nullptr || workspace_bytes < need)
     return fail(ATTNRES_ERR_ARG, "workspace of %lld bytes is smaller than the %lld needed", (long long)workspace_bytes,

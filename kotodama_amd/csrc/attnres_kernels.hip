@@ -2405,6 +2405,28 @@ __device__ __forceinline__ void route_bwd_stream_body(const attnres_route_bwd_pa
 }
 
 
+// The workgroup's query-gradient partial row from its waves' sums in LDS
+// ([wave][chunk][half][lane]), added in wave order.
+template <int NCH>
+__device__ __forceinline__ void rows_query_partial(const float4* dq_lds, float* part, int d, int nchunk) {
+  constexpr int ROW4 = NCH * 2 * 64;
+  float4* prow = reinterpret_cast<float4*>(part + (int64_t)blockIdx.x * d);
+  for (int j = threadIdx.x; j < ROW4; j += 64 * ATTNRES_BWD_ROWS_WAVES) {
+    const int c = j >> 7, h = (j >> 6) & 1, l = j & 63;
+    if (c * 64 + l >= nchunk) continue;
+    float4 a = dq_lds[j];
+#pragma unroll
+    for (int w = 1; w < ATTNRES_BWD_ROWS_WAVES; ++w) {
+      const float4 b = dq_lds[w * ROW4 + j];
+      a.x += b.x;
+      a.y += b.y;
+      a.z += b.z;
+      a.w += b.w;
+    }
+    prow[(c * 64 + l) * 2 + h] = a;
+  }
+}
+
 // ------------------------------- row-per-wave backward of narrow rows --
 //
 // The routing backward for bf16 sources and output gradients with rows of up
@@ -2609,21 +2631,7 @@ __device__ __forceinline__ void route_bwd_rows_body(const attnres_route_bwd_para
           make_float4(dq[c][4 * h], dq[c][4 * h + 1], dq[c][4 * h + 2], dq[c][4 * h + 3]);
   }
   __syncthreads();
-  float4* prow = reinterpret_cast<float4*>(P.dqw_part + (int64_t)blockIdx.x * P.d);
-  for (int j = tid; j < ROW4; j += 64 * ATTNRES_BWD_ROWS_WAVES) {
-    const int c = j >> 7, h = (j >> 6) & 1, l = j & 63;
-    if (c * 64 + l >= P.nchunk) continue;
-    float4 a = dq_lds[j];
-#pragma unroll
-    for (int w = 1; w < ATTNRES_BWD_ROWS_WAVES; ++w) {
-      const float4 b = dq_lds[w * ROW4 + j];
-      a.x += b.x;
-      a.y += b.y;
-      a.z += b.z;
-      a.w += b.w;
-    }
-    prow[(c * 64 + l) * 2 + h] = a;
-  }
+  rows_query_partial<NCH>(dq_lds, P.dqw_part, P.d, P.nchunk);
 }
 
 
@@ -3115,7 +3123,15 @@ __device__ __forceinline__ void route_bwd_mq_body(const attnres_route_bwd_mq_par
 // lane's own G_q / qw_q at that element, four queries along k), the VALU
 // adds (sum_q c2_qs) x_s and each gradient row is written once.  c1 goes to
 // the workspace for the query-gradient pass (route_bwd_dqw_body).
-template <int S, int V, int NQ4>
+//
+// ROWS: rows of up to 128 chunks, one wave per row and four rows per workgroup
+// (V = 1 up to 64 chunks).  With a workgroup per row those rows ran one wave
+// per workgroup, and the staged queries' LDS (16 KiB at hidden 1024, 8 queries)
+// left nine waves per CU; four waves now share them and no barrier is left in
+// the row loop.  8192 rows, S = 3, Q = 6, hidden 1024: 68.8 -> 41.8 us; the whole
+// backward with the query gradients at Q = 8: hidden 512, S = 4 73.7 -> 63.9,
+// hidden 1024, S = 3 107.9 -> 86.2, S = 8 165 -> 157.
+template <int S, int V, int NQ4, bool ROWS = false>
 __device__ __forceinline__ void route_bwd_mqg_body(const attnres_route_bwd_mq_params& P) {
   constexpr int VEC = 8;
   constexpr int SEG = 8;                 // lanes per query in the softmax (S <= 8)
@@ -3134,8 +3150,9 @@ __device__ __forceinline__ void route_bwd_mqg_body(const attnres_route_bwd_mq_pa
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int block = P.block;
+  constexpr int RW = ATTNRES_BWD_ROWS_WAVES;
+  const int wave = ROWS ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
+  const int block = ROWS ? 64 * RW : P.block;
   const int nwaves = (block + 63) >> 6;
   const int nq = P.num_queries;
   const int nchunk = P.nchunk;
@@ -3145,7 +3162,7 @@ __device__ __forceinline__ void route_bwd_mqg_body(const attnres_route_bwd_mq_pa
   const u32x4* qrow[V];  // this thread's chunks of the staged queries: qrow[k][16 * q], q < NQ
 #pragma unroll
   for (int k = 0; k < V; ++k) {
-    chunk[k] = tid + k * block;
+    chunk[k] = ROWS ? lane + k * 64 : tid + k * block;
     qrow[k] = qg_lds + qslot(chunk[k] < nchunk ? chunk[k] : nchunk - 1);  // chunks past the end read zeros
   }
 
@@ -3185,12 +3202,14 @@ __device__ __forceinline__ void route_bwd_mqg_body(const attnres_route_bwd_mq_pa
       for (int k = 0; k < V; ++k) gq[q][k] = ld_row(rg, (uint32_t)chunk[k] * 16);
     }
   };
-  if ((int64_t)blockIdx.x < P.n_tokens) load_row(blockIdx.x);
+  const int64_t tok0 = ROWS ? (int64_t)blockIdx.x * RW + wave : (int64_t)blockIdx.x;
+  const int64_t step = ROWS ? (int64_t)gridDim.x * RW : (int64_t)gridDim.x;
+  if (tok0 < P.n_tokens) load_row(tok0);
 
   __syncthreads();
 
   int ph = 0;
-  for (int64_t tok = blockIdx.x; tok < P.n_tokens; tok += gridDim.x) {
+  for (int64_t tok = tok0; tok < P.n_tokens; tok += step) {
     // Lane-derived indices and addresses are recomputed per row from an
     // opaque copy of the lane id: hoisted out of the row loop they stayed
     // live across it and spilled.
@@ -3252,14 +3271,20 @@ __device__ __forceinline__ void route_bwd_mqg_body(const attnres_route_bwd_mq_pa
         }
         wave_reduce_to_lds<HB>(part, red[ph][wave] + NPA, lr);
       }
-      __syncthreads();
+      if constexpr (ROWS) {
+        // the wave's own LDS rows: only the order of its accesses
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      } else {
+        __syncthreads();
+      }
 
       // ---- softmax and coefficients, lane 8g + s ----
       const int q = q0 + sg;
       const bool slot = sg < 4 && ss < S && q < nq;
       float t_ss = 0.f, t_dot = 0.f, t_gx = 0.f;
       if (slot) {
-        for (int w = 0; w < nwaves; ++w) {
+        for (int w = ROWS ? wave : 0; w < (ROWS ? wave + 1 : nwaves); ++w) {
           if (g4 == 0) t_ss += red[ph][w][ss];
           t_dot += red[ph][w][S + sg * S + ss];
           t_gx += red[ph][w][NPA + sg * S + ss];
@@ -3276,7 +3301,7 @@ __device__ __forceinline__ void route_bwd_mqg_body(const attnres_route_bwd_mq_pa
       const float glse = slot && P.grad_lse != nullptr ? P.grad_lse[(int64_t)q * P.n_tokens + tok] : 0.f;
       const float c1l = slot ? wl * (glse + (t_gx - go)) * rl : 0.f;  // cancel first, then add glse
       c2acc += slot ? -c1l * ll * rl * P.inv_d : 0.f;
-      if (wave == 0 && slot) P.c1[(tok * nq + q) * S + ss] = c1l;
+      if ((ROWS || wave == 0) && slot) P.c1[(tok * nq + q) * S + ss] = c1l;
 
       // ---- A operands: source 4*ks + ai, queries q0 .. q0+3 along k ----
 #pragma unroll
@@ -3366,7 +3391,7 @@ __device__ __forceinline__ void route_bwd_mqg_body(const attnres_route_bwd_mq_pa
         }
       }
     }
-    if (tok + gridDim.x < P.n_tokens) load_row(tok + gridDim.x);
+    if (tok + step < P.n_tokens) load_row(tok + step);
   }
 }
 
@@ -3750,6 +3775,107 @@ __device__ __forceinline__ void merge_bwd_body(const attnres_merge_bwd_params& P
 #pragma unroll
     for (int e = 0; e < VEC; ++e) qrow[(int64_t)chunk[k] * VEC + e] = dqa[k][e];
   }
+}
+
+// The same for bf16 rows of up to 6 KiB (NCH = the row's KiB, rounded up), one
+// wave per token row: the partial, inter and gradient rows are requested
+// together through buffer resources of the row's bytes (chunks past the row
+// end read zeros, their stores are dropped), the three sums reduced over the
+// wave, no barrier; the waves' query-gradient sums are added at the end
+// through LDS in a fixed order.  Two 4-wave workgroups per CU up to 4 KiB rows
+// (one: 0-27% slower at 1 KiB, even above), one from 5 KiB (two: 4-6% slower).
+// Per call with the reduction against the workgroup per row: 8192 rows of 1 KiB
+// 19.4 -> 14.1 us, 2 KiB 26.2 -> 20.9, 4 KiB 39.9 -> 35.9, 6 KiB 53.5 -> 49.9
+// (5.0 TB/s); 1024 rows of 6 KiB 17.4 -> 13.8; 32768 of 2 KiB 77.7 -> 61.6.
+template <int NCH>
+__device__ __forceinline__ void merge_bwd_rows_body(const attnres_merge_bwd_params& P) {
+  constexpr int ROW4 = NCH * 2 * 64;  // float4 slots of one query-gradient row
+  __shared__ float4 dq_lds[ATTNRES_BWD_ROWS_WAVES * ROW4];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  float qw[NCH][8], dq[NCH][8];
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int i = c * 64 + lane;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) qw[c][e] = 0.f, dq[c][e] = 0.f;
+    if (i < P.nchunk) load_param<8>(P.query, (int64_t)i * 8, P.param_bf16, qw[c]);
+  }
+  const uint32_t n_tok = (uint32_t)P.n_tokens;
+  const uint32_t nw = gridDim.x * ATTNRES_BWD_ROWS_WAVES;
+  const uint32_t row_size = (uint32_t)P.d * 2;
+  const uint32_t lane_off = (uint32_t)lane * 16;
+  auto row_at = [&](const void* base, uint32_t t) {
+    return row_rsrc(const_cast<char*>(uniform_ptr(reinterpret_cast<uint64_t>(base) + (uint64_t)t * row_size)), row_size);
+  };
+  auto lane63 = [](float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+  };
+  for (uint32_t t = blockIdx.x * ATTNRES_BWD_ROWS_WAVES + (uint32_t)wave; t < n_tok; t += nw) {
+    t = __builtin_amdgcn_readfirstlane(t);
+    u32x4 p[NCH], x[NCH], g[NCH];
+    const __amdgpu_buffer_rsrc_t pr = row_at(P.partial, t), ir = row_at(P.inter, t), gr = row_at(P.grad_out, t);
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      p[c] = ld_row_nt(pr, lane_off + (uint32_t)(c * 1024));
+      x[c] = ld_row_nt(ir, lane_off + (uint32_t)(c * 1024));
+      g[c] = ld_row_nt(gr, lane_off + (uint32_t)(c * 1024));
+    }
+    const float lse = ld_scalar_f32(P.inter_lse + t);
+    float ss = 0.f, dt = 0.f, ga = 0.f;
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float p0 = bf_lo(p[c][w]), p1 = bf_hi(p[c][w]);
+        ss = dot2_bf16(p[c][w], p[c][w], ss);
+        dt = __builtin_fmaf(p0, qw[c][2 * w], dt);
+        dt = __builtin_fmaf(p1, qw[c][2 * w + 1], dt);
+        ga = __builtin_fmaf(bf_lo(g[c][w]), p0 - bf_lo(x[c][w]), ga);
+        ga = __builtin_fmaf(bf_hi(g[c][w]), p1 - bf_hi(x[c][w]), ga);
+      }
+    }
+    const float tss = lane63(wave_sum_to_lane63(ss)), tdt = lane63(wave_sum_to_lane63(dt)),
+                tga = lane63(wave_sum_to_lane63(ga));
+    const float r = __builtin_amdgcn_rsqf(tss * P.inv_d + P.eps);
+    const float logit = tdt * r;
+    // pi and 1 - pi each from its own exponential (see merge_bwd_body)
+    const float z = logit - lse;
+    const float pi = 1.0f / (1.0f + __expf(-z));
+    const float qi = 1.0f / (1.0f + __expf(z));
+    const float gl = pi * qi * tga;
+    if (lane == 0 && P.grad_lse) P.grad_lse[t] = -gl;
+    const float cq = gl * r;
+    const float cp = -gl * logit * r * r * P.inv_d;
+    const __amdgpu_buffer_rsrc_t dpr = row_at(P.grad_partial, t), dir = row_at(P.grad_inter, t);
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      asm volatile("" : "+v"(p[c]), "+v"(g[c]));
+      u32x4 dp, di;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float p0 = bf_lo(p[c][w]), p1 = bf_hi(p[c][w]);
+        const float g0 = bf_lo(g[c][w]), g1 = bf_hi(g[c][w]);
+        dp[w] = pack_bf16(__builtin_fmaf(cp, p0, __builtin_fmaf(cq, qw[c][2 * w], pi * g0)),
+                          __builtin_fmaf(cp, p1, __builtin_fmaf(cq, qw[c][2 * w + 1], pi * g1)));
+        di[w] = pack_bf16(qi * g0, qi * g1);
+        dq[c][2 * w] = __builtin_fmaf(cq, p0, dq[c][2 * w]);
+        dq[c][2 * w + 1] = __builtin_fmaf(cq, p1, dq[c][2 * w + 1]);
+      }
+      st_row_nt(dpr, lane_off + (uint32_t)(c * 1024), dp);
+      st_row_nt(dir, lane_off + (uint32_t)(c * 1024), di);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      dq_lds[wave * ROW4 + (c * 2 + h) * 64 + lane] =
+          make_float4(dq[c][4 * h], dq[c][4 * h + 1], dq[c][4 * h + 2], dq[c][4 * h + 3]);
+  }
+  __syncthreads();
+  rows_query_partial<NCH>(dq_lds, P.dq_part, P.d, P.nchunk);
 }
 
 // Stage 1 of the query-gradient reduction: workgroup (x, y) sums partial
@@ -4216,6 +4342,20 @@ BWD_DQW(bf, true, 1) BWD_DQW(bf, true, 2) BWD_DQW(f32, false, 1) BWD_DQW(f32, fa
       attnres_route_bwd_mqg_s##S##_q##NQ4(attnres_route_bwd_mq_params P) {                      \
     route_bwd_mqg_body<S, 2, NQ4>(P);                                                           \
   }
+#define BWD_MQG_ROWS_ONE(S, V, NQ4)                                                             \
+  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_BWD_ROWS_WAVES)                     \
+      __attribute__((amdgpu_waves_per_eu(MQG_ROWS_EU(S, V, NQ4))))                              \
+      attnres_route_bwd_mqg_rows_v##V##_s##S##_q##NQ4(attnres_route_bwd_mq_params P) {          \
+    route_bwd_mqg_body<S, V, NQ4, true>(P);                                                     \
+  }
+// Waves per SIMD by the registers of a row: S + 4 NQ4 rows of 4 V, the A
+// operands (16 NQ4 per four sources) and about 60.
+#ifndef MQG_ROWS_EU
+#define MQG_ROWS_REGS(S, V, NQ4) (4 * (V) * ((S) + 4 * (NQ4)) + 8 * (NQ4) * (((S) + 3) / 4) + 60)
+#define MQG_ROWS_EU(S, V, NQ4) (MQG_ROWS_REGS(S, V, NQ4) <= 128 ? 4 : MQG_ROWS_REGS(S, V, NQ4) <= 168 ? 3 : 2)
+#endif
+#define BWD_MQG_ROWS(S) \
+  BWD_MQG_ROWS_ONE(S, 1, 1) BWD_MQG_ROWS_ONE(S, 1, 2) BWD_MQG_ROWS_ONE(S, 2, 1) BWD_MQG_ROWS_ONE(S, 2, 2)
 #define BWD_DQWM(V)                                                                             \
   extern "C" __global__ void __launch_bounds__(512) attnres_route_bwd_dqwm_bf_v##V(             \
       attnres_route_bwd_dqw_params P) {                                                         \
@@ -4223,6 +4363,8 @@ BWD_DQW(bf, true, 1) BWD_DQW(bf, true, 2) BWD_DQW(f32, false, 1) BWD_DQW(f32, fa
   }
 #if ATTNRES_PART == 7 || defined(ATTNRES_ALL_PARTS)
 BWD_DQWM(1) BWD_DQWM(2)
+BWD_MQG_ROWS(1) BWD_MQG_ROWS(2) BWD_MQG_ROWS(3) BWD_MQG_ROWS(4)
+BWD_MQG_ROWS(5) BWD_MQG_ROWS(6) BWD_MQG_ROWS(7) BWD_MQG_ROWS(8)
 BWD_MQG(1, 1) BWD_MQG(2, 1) BWD_MQG(3, 1) BWD_MQG(4, 1) BWD_MQG(5, 1) BWD_MQG(6, 1) BWD_MQG(7, 1) BWD_MQG(8, 1)
 BWD_MQG(1, 2) BWD_MQG(2, 2) BWD_MQG(3, 2) BWD_MQG(4, 2) BWD_MQG(5, 2) BWD_MQG(6, 2) BWD_MQG(7, 2) BWD_MQG(8, 2)
 #endif
@@ -4317,12 +4459,19 @@ BWD_STREAM_ONE_DEFER(8, 8, 2) BWD_STREAM_ONE_DEFER(9, 8, 3)
       attnres_route_bwd_rows_c##NCH##_s##S##_defer(attnres_route_bwd_params P) {                         \
     route_bwd_rows_body<S, NCH, true, true>(P);                                                          \
   }
+#define MERGE_BWD_ROWS(NCH)                                                                              \
+  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_BWD_ROWS_WAVES)                              \
+      __attribute__((amdgpu_waves_per_eu(BWD_ROWS_EU(0, NCH, 3))))                                       \
+      attnres_merge_bwd_rows_c##NCH(attnres_merge_bwd_params P) {                                        \
+    merge_bwd_rows_body<NCH>(P);                                                                         \
+  }
 #define BWD_ROWS_S(S) \
   BWD_ROWS_ONE(S, 1) BWD_ROWS_ONE(S, 2) BWD_ROWS_ONE(S, 3) BWD_ROWS_ADD(S, 1) BWD_ROWS_ADD(S, 2)
 #if ATTNRES_PART == 11 || defined(ATTNRES_ALL_PARTS)
 BWD_ROWS_S(1) BWD_ROWS_S(2) BWD_ROWS_S(3) BWD_ROWS_S(4) BWD_ROWS_S(5)
 BWD_ROWS_S(6) BWD_ROWS_S(7) BWD_ROWS_S(8) BWD_ROWS_S(9)
 BWD_ROWS_ADD(1, 3) BWD_ROWS_ADD(2, 3) BWD_ROWS_ADD(3, 3) BWD_ROWS_ADD(4, 3) BWD_ROWS_ADD(5, 3) BWD_ROWS_ADD(6, 3)
+MERGE_BWD_ROWS(1) MERGE_BWD_ROWS(2) MERGE_BWD_ROWS(3) MERGE_BWD_ROWS(4) MERGE_BWD_ROWS(5) MERGE_BWD_ROWS(6)
 BWD_ROWS_DEFER(2, 1) BWD_ROWS_DEFER(3, 1) BWD_ROWS_DEFER(4, 1) BWD_ROWS_DEFER(5, 1)
 BWD_ROWS_DEFER(6, 1) BWD_ROWS_DEFER(7, 1) BWD_ROWS_DEFER(8, 1)
 BWD_ROWS_DEFER(2, 2) BWD_ROWS_DEFER(3, 2) BWD_ROWS_DEFER(4, 2) BWD_ROWS_DEFER(5, 2)

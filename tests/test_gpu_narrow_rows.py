@@ -6,10 +6,11 @@ import pytest
 import torch
 
 import kotodama_amd
-from kotodama_amd import _capi
+from kotodama_amd import _capi, ops
+from oracle import attnres_oracle as O
 
 from .test_gpu_accumulate import _call, _case
-from .test_gpu_backward import Norm, _bwd_kernel_name, check_grad, make_case, oracle_grads
+from .test_gpu_backward import Norm, _bwd_kernel_name, bwd_queries_kernel, check_grad, make_case, np64, oracle_grads
 
 pytestmark = pytest.mark.gpu
 
@@ -89,3 +90,53 @@ def test_cached_and_streamed_sources_agree(gpu, D, S, lo, hi):
         small = kotodama_amd.route_static(buf[:, :lo].contiguous(), query, norm, mask, S)
         large = kotodama_amd.route_static(buf, query, norm, mask, S)
     assert torch.equal(small, large[:lo])
+
+
+MERGE_CASES = [(8, 5, None), (504, 1100, None), (520, 2049, torch.float32), (1536, 1027, None), (2560, 1025, None),
+               (3072, 3, None)]
+
+
+@pytest.mark.parametrize("D,N,qd", MERGE_CASES, ids=[f"D{c[0]}-N{c[1]}{'-qf32' if c[2] else ''}" for c in MERGE_CASES])
+def test_row_per_wave_merge_backward_matches_oracle(gpu, D, N, qd):
+    print(f"row-per-wave merge backward D={D} N={N} query={qd}", flush=True)
+    g = torch.Generator(device="cpu").manual_seed(D + N)
+    p, inter = ((torch.randn(1, N, D, generator=g) * s).to(torch.bfloat16).to(gpu).requires_grad_() for s in (2, 1))
+    q = (torch.randn(D, generator=g) * 0.1).to(qd or torch.bfloat16).to(gpu).requires_grad_()
+    lse = torch.randn(1, N, generator=g).to(gpu).requires_grad_()
+    G = torch.randn(1, N, D, generator=g).to(torch.bfloat16).to(gpu)
+    prev = _capi.set_kernel_policy(_capi.POLICY_STREAM)
+    try:
+        out = ops.merge_call(p, q, inter, lse, 1e-5)
+        out.backward(G)
+        torch.cuda.synchronize()
+    finally:
+        _capi.set_kernel_policy(prev)
+    b = O.merge_backward(np64(p).reshape(N, D), np64(q), np64(inter).reshape(N, D), np64(lse).reshape(N), 1e-5,
+                         np64(G).reshape(N, D))
+    check_grad(p.grad.reshape(N, D), b["dpartial"], torch.bfloat16, "dpartial")
+    check_grad(inter.grad.reshape(N, D), b["dinter"], torch.bfloat16, "dinter")
+    check_grad(lse.grad.reshape(N), b["dlse"], torch.float32, "dlse")
+    check_grad(q.grad, b["dq"], q.dtype, "dquery")
+
+
+QUERY_CASES = [(8, 3, 5, 2), (504, 8, 1030, 8), (520, 5, 1027, 5), (1024, 3, 1025, 6), (1016, 1, 2, 8)]
+
+
+@pytest.mark.parametrize("D,S,N,Q", QUERY_CASES, ids=[f"D{c[0]}-S{c[1]}-N{c[2]}-Q{c[3]}" for c in QUERY_CASES])
+def test_row_per_wave_batched_backward_matches_oracle(gpu, D, S, N, Q):
+    print(f"row-per-wave batched backward D={D} S={S} N={N} Q={Q}", flush=True)
+    v = 1 if D <= 512 else 2
+    assert bwd_queries_kernel(S, D, torch.bfloat16, Q) == f"attnres_route_bwd_mqg_rows_v{v}_s{S}_q{(Q + 3) // 4}"
+    g = torch.Generator(device="cpu").manual_seed(D + S + N)
+    buf = torch.randn(S, 1, N, D, generator=g).to(torch.bfloat16).to(gpu).requires_grad_()
+    qs = (torch.randn(Q, D, generator=g) * 0.05).to(torch.bfloat16).to(gpu).requires_grad_()
+    G = torch.randn(Q, 1, N, D, generator=g).to(torch.bfloat16).to(gpu)
+    GL = torch.randn(Q, 1, N, generator=g).to(gpu)
+    out, _, lse, _, _ = ops.route_call(buf, S, qs, None, 1e-5, torch.bfloat16, want_lse=True)
+    torch.autograd.backward([out, lse], [G, GL])
+    x, dx = np64(buf).reshape(S, N, D), 0
+    for j in range(Q):
+        b = O.route_backward(x, np64(qs[j]), 1e-5, np64(G[j]).reshape(N, D), np64(GL[j]).reshape(N))
+        dx = dx + b["dx"]
+        check_grad(qs.grad[j], b["dqw"], torch.bfloat16, f"dquery[{j}]")
+    check_grad(buf.grad.reshape(S, N, D), dx, torch.bfloat16, "dsources")
