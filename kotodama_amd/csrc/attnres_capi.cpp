@@ -115,6 +115,7 @@ struct DeviceState {
   KernelSlot merge_bwd_rows[6];  // its row-per-wave form: row KiB (1..6)
   KernelSlot bwd_mq[kBwdFuncs];  // batched-query backward: (source, grad_out) dtypes x S x V
   KernelSlot bwd_dqw[4];         // source dtype x V
+  KernelSlot bwd_dqw_grouped;    // bf16, one chunk per thread, several row groups per workgroup
   KernelSlot bwd_mqg_rows[2 * 2 * 9];  // its row-per-wave form: chunks per lane x query groups x S
   KernelSlot bwd_mqg[2 * 9];     // batched-query backward on the matrix cores: query groups x S
   KernelSlot bwd_defer[2 * 10];  // row-per-wave backward with deferred block gradients: 6 / 8 KiB rows x S
@@ -526,15 +527,17 @@ int get_bwd_mq(DeviceState& st, bool bf, bool gbf, int s, int v, int block, hipF
 }
 
 // bf16 sources: the matrix-core variant (part 7) unless ATTNRES_MQG=0.
-int get_bwd_dqw(DeviceState& st, bool bf, int v, int block, hipFunction_t* f, int* bpc) {
+int get_bwd_dqw(DeviceState& st, bool bf, int v, int block, bool grouped, size_t lds, hipFunction_t* f, int* bpc) {
   char name[96];
+  if (grouped)
+    return slot_get(st, st.bwd_dqw_grouped, kBwdMqgPart, "attnres_route_bwd_dqwm_grouped_bf_v1", block, lds, f, bpc);
   const bool mfma = bf && tuning().mqg != 0;
   if (mfma) {
     snprintf(name, sizeof(name), "attnres_route_bwd_dqwm_bf_v%d", v);
   } else {
     snprintf(name, sizeof(name), "attnres_route_bwd_dqw_%s_v%d", bf ? "bf" : "f32", v);
   }
-  return slot_get(st, st.bwd_dqw[(bf ? 0 : 2) + (v - 1)], mfma ? kBwdMqgPart : kBwdMqPart, name, block, 0, f, bpc);
+  return slot_get(st, st.bwd_dqw[(bf ? 0 : 2) + (v - 1)], mfma ? kBwdMqgPart : kBwdMqPart, name, block, lds, f, bpc);
 }
 
 // Batched-query backward on the matrix cores (code-object part 7): bf16
@@ -979,8 +982,12 @@ int reduce_launch(const ReduceFns& fn, void* workspace, int nparts, int hidden, 
   // one launch (32 columns per 1024-thread workgroup) for up to four queries
   // where its byte offsets, up to 1024 rows past the last partial row, fit in
   // 32 bits; else two
-  if (!tuning().reduce_two_stage && num_queries <= 4 && (int64_t)(nparts + 1024) * width * 4 < (int64_t)1 << 32)
-    return launch(fn.cols, (hidden + 31) / 32, 1024, R, stream);
+  const bool fits = (int64_t)(nparts + 1024) * width * 4 < (int64_t)1 << 32;
+  if (!tuning().reduce_two_stage && fits) {
+    // without a gain gradient the queries are independent: one per workgroup
+    if (num_queries > 1 && grad_gain == nullptr) return launch(fn.cols, (hidden + 31) / 32, 1024, R, stream, num_queries);
+    if (num_queries <= 4) return launch(fn.cols, (hidden + 31) / 32, 1024, R, stream);
+  }
   if (nparts > 64) {
     int rc = launch(fn.stage, (int)((width + 63) / 64), 256, R, stream, (nparts + 63) / 64);
     if (rc != ATTNRES_OK) return rc;
@@ -1808,14 +1815,30 @@ int attnres_route_bwd_queries(const void* const* sources, int num_sources, int64
   ReduceFns redfns;
   const ReduceFns* red = nullptr;
   int64_t grid_q = 0;
+  int dqw_groups = 1;
+  size_t dqw_lds = 0;
   if (want_q) {
-    rc = get_bwd_dqw(*st, bf, v, block, &fq, &bpcq);
+    // the matrix-core pass: up to four row groups in a workgroup of at most 512
+    // threads, so that one workgroup per CU (two of up to 256 threads) keeps
+    // enough rows in flight; rows too wide for two groups run two per CU, or one
+    // over up to 16 rows per CU (hidden 3072, Q = 8: 1000 rows at S = 4 58.4
+    // against 52.2 us; at 8192 rows 3% faster at S = 4 and 1% slower at S = 7, at
+    // 32768 the pass alone 20% slower)
+    int per_cu_q = kBwdDqwPerCu;
+    if (bf && tuning().mqg != 0 && v == 1) {
+      dqw_groups = kMaxThreads / block < 4 ? kMaxThreads / block : 4;
+      const int ng = num_queries < 8 ? num_queries : 8;
+      if (dqw_groups > 1) dqw_lds = (size_t)ng * (size_t)nchunk * 8 * sizeof(float);
+      if (dqw_groups > 1 ? block * dqw_groups > 256 : num_tokens <= 16LL * st->num_cus) per_cu_q = 1;
+    }
+    rc = get_bwd_dqw(*st, bf, v, block * dqw_groups, dqw_groups > 1, dqw_lds, &fq, &bpcq);
     if (rc != ATTNRES_OK) return rc;
     rc = get_reduce(*st, &redfns);
     red = &redfns;
     if (rc != ATTNRES_OK) return rc;
-    grid_q = (int64_t)st->num_cus * (bpcq < kBwdDqwPerCu ? bpcq : kBwdDqwPerCu);
-    if (grid_q > num_tokens) grid_q = num_tokens;
+    grid_q = (int64_t)st->num_cus * (bpcq < per_cu_q ? bpcq : per_cu_q);
+    const int64_t row_groups = (num_tokens + dqw_groups - 1) / dqw_groups;
+    if (grid_q > row_groups) grid_q = row_groups;
   }
   const int64_t c1_bytes = bwd_mq_c1_bytes(num_tokens, num_sources, num_queries);
   const int64_t need = c1_bytes + grid_q * (int64_t)num_queries * hidden * (int64_t)sizeof(float);
@@ -1873,7 +1896,7 @@ int attnres_route_bwd_queries(const void* const* sources, int num_sources, int64
   Q.block = block;
   for (int q0 = 0; q0 < num_queries; q0 += 8) {  // eight queries per pass over the sources
     Q.q0 = q0;
-    rc = launch(fq, (int)grid_q, block, Q, stream);
+    rc = launch(fq, (int)grid_q, block * dqw_groups, Q, stream, 1, dqw_lds);
     if (rc != ATTNRES_OK) return rc;
   }
   return reduce_launch(*red, part, (int)grid_q, hidden, query, gain, param_dtype, grad_query, grad_gain, stream,

@@ -3483,12 +3483,23 @@ __device__ __forceinline__ void route_bwd_dqw_body(const attnres_route_bwd_dqw_p
 // and c1 values are requested before the current four's 2 * 2 MFMAs per
 // element (two query groups, hi and lo).  Slots past the last pair read
 // through a zero-byte buffer resource: zeros, no memory traffic.
-template <int V>
+//
+// GROUPED: P.block threads per row and as many row groups as the workgroup
+// holds, their sums added through LDS in group order, so that narrow rows keep
+// more waves per CU and write fewer partial rows (512 workgroups of one or two
+// waves before).  With the queries reduced side by side, 8192 rows, the whole
+// batched backward: hidden 512, S = 7, Q = 8 87.4 -> 67.8 us, hidden 1024,
+// S = 3, Q = 6 77.1 -> 65.8.
+template <int V, bool GROUPED>
 __device__ __forceinline__ void route_bwd_dqwm_body(const attnres_route_bwd_dqw_params& P) {
   constexpr int NQ4 = 2;  // eight queries per pass
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int block = P.block;
+  extern __shared__ float4 dqw_lds[];  // with more than one row group: [query][chunk][half] sums
+  const int block = P.block;  // threads per row
+  const int groups = GROUPED ? (int)blockDim.x / block : 1;  // rows in flight per workgroup
+  const int group = GROUPED ? (int)threadIdx.x / block : 0;
+  const int tid = (int)threadIdx.x - group * block;
+  const int lane = (int)threadIdx.x & 63;
+  const int64_t row0 = (int64_t)blockIdx.x * groups + group, row_step = (int64_t)gridDim.x * groups;
   const int S = P.num_sources;
   const int nq = P.num_queries;
   const int q0 = P.q0;
@@ -3513,18 +3524,19 @@ __device__ __forceinline__ void route_bwd_dqwm_body(const attnres_route_bwd_dqw_
   }
   const int64_t row_bytes_ld = P.src_ld * 2;
   const uint32_t row_bytes = (uint32_t)(P.d * 2);
-  const uint32_t rows =
-      (int64_t)blockIdx.x < P.n_tokens ? (uint32_t)((P.n_tokens - 1 - blockIdx.x) / gridDim.x + 1) : 0u;
+  uint32_t rows = row0 < P.n_tokens ? (uint32_t)((P.n_tokens - 1 - row0) / row_step + 1) : 0u;
+  if constexpr (GROUPED) rows = __builtin_amdgcn_readfirstlane(rows);
   const uint32_t npairs = rows * (uint32_t)S;
   const uint32_t items = (npairs + 3) / 4;
 
-  // the next pair to request: row blockIdx.x + pj * gridDim.x, source ps
+  // the next pair to request: row row0 + pj * row_step, source ps
   uint32_t pj = 0, ps = 0, pnext = 0;
   auto load_item = [&](u32x4 (&x)[4][V], float (&c)[NQ4][4]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const bool valid = pnext < npairs;
-      const int64_t tok = (int64_t)blockIdx.x + (int64_t)pj * gridDim.x;
+      int64_t tok = row0 + (int64_t)pj * row_step;
+      if constexpr (GROUPED) tok = uniform_i64(tok);
       char* row = reinterpret_cast<char*>(const_cast<void*>(P.src[ps])) + tok * row_bytes_ld;
       const __amdgpu_buffer_rsrc_t rs = row_rsrc(row, valid ? row_bytes : 0u);
 #pragma unroll
@@ -3583,20 +3595,62 @@ __device__ __forceinline__ void route_bwd_dqwm_body(const attnres_route_bwd_dqw_
     }
   }
   float* prow = P.part + (int64_t)blockIdx.x * nq * P.d;
+  auto piece = [&](int k, int g4, int i, int h) {
+    return make_float4(acc[k][4 * h][g4][i], acc[k][4 * h + 1][g4][i], acc[k][4 * h + 2][g4][i],
+                       acc[k][4 * h + 3][g4][i]);
+  };
+  if constexpr (!GROUPED) {
 #pragma unroll
-  for (int k = 0; k < V; ++k) {
-    if (!ok[k]) continue;
+    for (int k = 0; k < V; ++k) {
+      if (!ok[k]) continue;
 #pragma unroll
-    for (int g4 = 0; g4 < NQ4; ++g4) {
+      for (int g4 = 0; g4 < NQ4; ++g4) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int g = 4 * g4 + i;
-        if (g >= ng) continue;
-        float4* dst = reinterpret_cast<float4*>(prow + (int64_t)(q0 + g) * P.d + (int64_t)chunk[k] * 8);
-        dst[0] = make_float4(acc[k][0][g4][i], acc[k][1][g4][i], acc[k][2][g4][i], acc[k][3][g4][i]);
-        dst[1] = make_float4(acc[k][4][g4][i], acc[k][5][g4][i], acc[k][6][g4][i], acc[k][7][g4][i]);
+        for (int i = 0; i < 4; ++i) {
+          const int g = 4 * g4 + i;
+          if (g >= ng) continue;
+          float4* dst = reinterpret_cast<float4*>(prow + (int64_t)(q0 + g) * P.d + (int64_t)chunk[k] * 8);
+          dst[0] = piece(k, g4, i, 0);
+          dst[1] = piece(k, g4, i, 1);
+        }
       }
     }
+    return;
+  }
+  // the row groups' sums through LDS, added in group order
+  for (int r = 0; r < groups; ++r) {
+    if (r == group) {
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        if (!ok[k]) continue;
+#pragma unroll
+        for (int g4 = 0; g4 < NQ4; ++g4) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int g = 4 * g4 + i;
+            if (g >= ng) continue;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              float4* at = dqw_lds + (g * 2 + h) * P.nchunk + chunk[k];
+              float4 v = piece(k, g4, i, h);
+              if (r > 0) {
+                const float4 t = *at;
+                v.x += t.x;
+                v.y += t.y;
+                v.z += t.z;
+                v.w += t.w;
+              }
+              *at = v;
+            }
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+  for (int j = threadIdx.x; j < ng * 2 * P.nchunk; j += (int)blockDim.x) {
+    const int c = j / 2 % P.nchunk, g = j / 2 / P.nchunk, h = j & 1;
+    reinterpret_cast<float4*>(prow + (int64_t)(q0 + g) * P.d)[c * 2 + h] = dqw_lds[(g * 2 + h) * P.nchunk + c];
   }
 }
 
@@ -3927,7 +3981,9 @@ __device__ __forceinline__ void reduce_dqw_cols_body(const attnres_reduce_params
   if (P.gain && in) g = P.param_bf16 ? bf_lo(reinterpret_cast<const uint16_t*>(P.gain)[col])
                                      : reinterpret_cast<const float*>(P.gain)[col];
   float dg = 0.f;
-  for (int q0 = 0; q0 < nq; q0 += QB) {
+  // gridDim.y > 1 (no gain gradient): one query per workgroup, else all in turn
+  const int qfirst = gridDim.y > 1 ? (int)blockIdx.y : 0, qlast = gridDim.y > 1 ? qfirst + 1 : nq;
+  for (int q0 = qfirst; q0 < qlast; q0 += QB) {
     float acc[QB];
 #pragma unroll
     for (int b = 0; b < QB; ++b) acc[b] = 0.f;
@@ -4359,10 +4415,15 @@ BWD_DQW(bf, true, 1) BWD_DQW(bf, true, 2) BWD_DQW(f32, false, 1) BWD_DQW(f32, fa
 #define BWD_DQWM(V)                                                                             \
   extern "C" __global__ void __launch_bounds__(512) attnres_route_bwd_dqwm_bf_v##V(             \
       attnres_route_bwd_dqw_params P) {                                                         \
-    route_bwd_dqwm_body<V>(P);                                                                  \
+    route_bwd_dqwm_body<V, false>(P);                                                           \
+  }
+#define BWD_DQWM_GROUPED(V)                                                                     \
+  extern "C" __global__ void __launch_bounds__(512) attnres_route_bwd_dqwm_grouped_bf_v##V(     \
+      attnres_route_bwd_dqw_params P) {                                                         \
+    route_bwd_dqwm_body<V, true>(P);                                                            \
   }
 #if ATTNRES_PART == 7 || defined(ATTNRES_ALL_PARTS)
-BWD_DQWM(1) BWD_DQWM(2)
+BWD_DQWM(1) BWD_DQWM(2) BWD_DQWM_GROUPED(1)
 BWD_MQG_ROWS(1) BWD_MQG_ROWS(2) BWD_MQG_ROWS(3) BWD_MQG_ROWS(4)
 BWD_MQG_ROWS(5) BWD_MQG_ROWS(6) BWD_MQG_ROWS(7) BWD_MQG_ROWS(8)
 BWD_MQG(1, 1) BWD_MQG(2, 1) BWD_MQG(3, 1) BWD_MQG(4, 1) BWD_MQG(5, 1) BWD_MQG(6, 1) BWD_MQG(7, 1) BWD_MQG(8, 1)
