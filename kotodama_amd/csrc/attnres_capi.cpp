@@ -941,7 +941,12 @@ int route_launch(const void* const* sources, int num_sources, int64_t num_tokens
   P.num_sources = num_sources;
   P.block = block;
   P.out_batch = out_batch;
-  P.src_cached = num_sources * num_tokens * (int64_t)hidden * esize(src_dtype) <= kCachedSourceBytes;
+  // The batched-query kernel reads rows of more than 128 chunks through the
+  // caches (with the hint hidden 2048 ran 2% slower, hidden 3072 at 300 rows 7%)
+  // and narrower ones with it: hidden 512, S = 4, Q = 8, 8192 rows 24.7 -> 22.9
+  // us, hidden 1000, S = 7, 16384 rows 119 -> 90.
+  P.src_cached = ch.qg_lds > 0 ? nchunk > 128
+                               : num_sources * num_tokens * (int64_t)hidden * esize(src_dtype) <= kCachedSourceBytes;
   P.eps = eps;
   P.inv_d = 1.0f / (float)hidden;
   // The streaming kernels run one 4-wave workgroup per CU from 6 KiB rows: at
