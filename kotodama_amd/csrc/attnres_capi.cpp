@@ -104,6 +104,7 @@ struct DeviceState {
   KernelSlot route_qg[kNumS * 2];  // batched-query kernels: S x V
   KernelSlot stream[kStreamFuncs];
   KernelSlot merge[kMergeFuncs];
+  KernelSlot merge_rows[3];  // row-per-wave merge of narrow rows: row KiB (1..3)
   KernelSlot merge_stream[2 * kStreamMaxChunks];  // row-per-wave merge: query path x row KiB
   KernelSlot bwd[kBwdFuncs];
   KernelSlot bwd_stream[2 * 10];  // row-per-wave backward: rows of 6 / 8 KiB x S (1..9)
@@ -360,6 +361,12 @@ int get_merge_stream(DeviceState& st, bool d2, int nch, hipFunction_t* f) {
   return slot_function(st, st.merge_stream[(d2 ? 0 : kStreamMaxChunks) + (nch - 1)], kMergePart, name, f);
 }
 
+int get_merge_rows(DeviceState& st, int nch, hipFunction_t* f, int* bpc) {
+  char name[96];
+  snprintf(name, sizeof(name), "attnres_merge_rows_c%d", nch);
+  return slot_get(st, st.merge_rows[nch - 1], kMergePart, name, 64 * ATTNRES_ROWS_WAVES, 0, f, bpc);
+}
+
 int get_merge(DeviceState& st, bool pbf, bool ibf, int v, int block, hipFunction_t* f, int* bpc) {
   char name[96];
   snprintf(name, sizeof(name), "attnres_merge_%s_%s_v%d", pbf ? "bf" : "f32", ibf ? "bf" : "f32", v);
@@ -447,12 +454,12 @@ int get_bwd_rows(DeviceState& st, int nch, int s, BwdRowsVariant var, hipFunctio
   char name[96];
   snprintf(name, sizeof(name), "attnres_route_bwd_rows_c%d_s%d%s", nch, s, suffix[var]);
   return slot_get(st, st.bwd_rows[((int)var * 3 + nch - 1) * 10 + s], kBwdRowsPart, name,
-                  64 * ATTNRES_BWD_ROWS_WAVES, 0, f, bpc);
+                  64 * ATTNRES_ROWS_WAVES, 0, f, bpc);
 }
 // Its grid: two workgroups per CU where they fit (measured in the kernel's comment).
 int bwd_rows_grid(int64_t num_tokens, int num_cus, int bpc, int per_cu = 2) {
   const int limit = tuning().bwd_per_cu > 0 ? tuning().bwd_per_cu : per_cu;
-  const int64_t need = (num_tokens + ATTNRES_BWD_ROWS_WAVES - 1) / ATTNRES_BWD_ROWS_WAVES;
+  const int64_t need = (num_tokens + ATTNRES_ROWS_WAVES - 1) / ATTNRES_ROWS_WAVES;
   const int64_t cap = (int64_t)num_cus * (bpc < limit ? bpc : limit);
   return (int)(need < cap ? need : cap);
 }
@@ -565,7 +572,7 @@ int get_bwd_mqg_rows(DeviceState& st, int v, int s, int nq4, size_t lds, hipFunc
   char name[96];
   snprintf(name, sizeof(name), "attnres_route_bwd_mqg_rows_v%d_s%d_q%d", v, s, nq4);
   return slot_get(st, st.bwd_mqg_rows[((v - 1) * 2 + nq4 - 1) * 9 + s], kBwdMqgPart, name,
-                  64 * ATTNRES_BWD_ROWS_WAVES, lds, f, bpc);
+                  64 * ATTNRES_ROWS_WAVES, lds, f, bpc);
 }
 
 int get_merge_bwd(DeviceState& st, bool pbf, bool ibf, int v, int block, hipFunction_t* f, int* bpc) {
@@ -578,7 +585,7 @@ int get_merge_bwd(DeviceState& st, bool pbf, bool ibf, int v, int block, hipFunc
 int get_merge_bwd_rows(DeviceState& st, int nch, hipFunction_t* f, int* bpc) {
   char name[96];
   snprintf(name, sizeof(name), "attnres_merge_bwd_rows_c%d", nch);
-  return slot_get(st, st.merge_bwd_rows[nch - 1], kBwdRowsPart, name, 64 * ATTNRES_BWD_ROWS_WAVES, 0, f, bpc);
+  return slot_get(st, st.merge_bwd_rows[nch - 1], kBwdRowsPart, name, 64 * ATTNRES_ROWS_WAVES, 0, f, bpc);
 }
 // Row KiB (rounded up) of the merge backward's row-per-wave kernel (bf16 rows of
 // up to 6 KiB) for this call, or 0 for the row-per-workgroup one.  AUTO takes
@@ -791,11 +798,12 @@ constexpr int64_t kCachedSourceBytes = 24 << 20;
 // Shared validation + launch of the route kernel.  `mode`/`delta` are the
 // fused partial-update inputs of attnres_block_step.
 // The kernel choice of one merge call, shared by the launch and the name
-// query: the row-per-wave kernel for bf16 rows of whole 1 KiB chunks (at most
+// query: the narrow rows' kernel, the row-per-wave kernel for bf16 rows of whole 1 KiB chunks (at most
 // kStreamMaxChunks) over enough rows (the routing kernels' policy and
 // threshold), one workgroup of four waves per CU; else one workgroup per row.
 struct MergeChoice {
   bool stream = false;
+  bool rows = false;  // the narrow rows' kernel (nch: row KiB, rounded up)
   int nch = 0;    // row KiB (row-per-wave kernel)
   int v = 0;      // chunks per thread (row-per-workgroup kernel); 0: no launch shape
   int block = 0;  // threads per workgroup
@@ -811,6 +819,17 @@ MergeChoice plan_merge(int64_t num_tokens, int hidden, int partial_dtype, int in
   const int want_stream = policy == ATTNRES_POLICY_STREAM      ? 1
                           : policy == ATTNRES_POLICY_WORKGROUP ? 0
                                                                : tuning().stream;
+  // AUTO, rows of up to 3 KiB, from four rows per CU: against the kernels below
+  // it measured, per call, hidden 512 10.0 -> 6.3 us at 8192 rows and 31.5 ->
+  // 17.2 at 32768, hidden 1024 11.8 -> 9.9 and 38.1 -> 32.6, hidden 768 9.2 ->
+  // 8.2, hidden 1536 15.2 -> 13.7; at 300 rows 1-8% slower, at 4 KiB rows even.
+  ch.rows = want_stream < 0 && pbf && ibf && hidden <= 1536 && num_tokens >= 4LL * st.num_cus &&
+            num_tokens < (int64_t)1 << 31;
+  if (ch.rows) {
+    ch.nch = (hidden + 511) / 512;
+    ch.block = 64 * ATTNRES_ROWS_WAVES;
+    return ch;
+  }
   ch.stream = stream_shape && (want_stream == 1 || (want_stream < 0 && num_tokens >= tuning().stream_min_tokens));
   if (ch.stream) {
     ch.block = 64 * (tuning().stream_waves > 0 ? tuning().stream_waves : kStreamWaves);
@@ -1056,7 +1075,9 @@ int attnres_merge_kernel_name(int64_t num_tokens, int hidden, int partial_dtype,
   int rc = ensure_loaded(&st);
   if (rc != ATTNRES_OK) return rc;
   const MergeChoice ch = plan_merge(num_tokens, hidden, partial_dtype, inter_dtype, *st);
-  if (ch.stream) {
+  if (ch.rows) {
+    snprintf(buf, (size_t)buf_len, "attnres_merge_rows_c%d", ch.nch);
+  } else if (ch.stream) {
     snprintf(buf, (size_t)buf_len, "attnres_merge_stream_%s_c%d", param_dtype == ATTNRES_DTYPE_BF16 ? "d2" : "fm",
              ch.nch);
   } else if (ch.v != 0) {
@@ -1182,12 +1203,14 @@ int attnres_merge_fwd(const void* partial, int64_t num_tokens, int hidden, int p
   int rc = ensure_loaded(&st);
   if (rc != ATTNRES_OK) return rc;
   const MergeChoice ch = plan_merge(num_tokens, hidden, partial_dtype, inter_dtype, *st);
-  if (!ch.stream && ch.v == 0) return fail(ATTNRES_ERR_UNSUPPORTED, "hidden=%d has no launch shape", hidden);
+  if (!ch.rows && !ch.stream && ch.v == 0)
+    return fail(ATTNRES_ERR_UNSUPPORTED, "hidden=%d has no launch shape", hidden);
   const bool use_stream = ch.stream;
   const int block = ch.block;
   hipFunction_t f = nullptr;
   int bpc = 1;
-  rc = use_stream ? get_merge_stream(*st, param_dtype == ATTNRES_DTYPE_BF16, ch.nch, &f)
+  rc = ch.rows      ? get_merge_rows(*st, ch.nch, &f, &bpc)
+       : use_stream ? get_merge_stream(*st, param_dtype == ATTNRES_DTYPE_BF16, ch.nch, &f)
                   : get_merge(*st, pbf, ibf, ch.v, block, &f, &bpc);
   if (rc != ATTNRES_OK) return rc;
 
@@ -1211,6 +1234,12 @@ int attnres_merge_fwd(const void* partial, int64_t num_tokens, int hidden, int p
   P.block = block;
   P.eps = eps;
   P.inv_d = 1.0f / (float)hidden;
+  if (ch.rows) {
+    constexpr int per_cu = 3;  // two to eight within 3%, one 10-50% slower
+    const int64_t need = (num_tokens + ATTNRES_ROWS_WAVES - 1) / ATTNRES_ROWS_WAVES;
+    const int64_t cap = (int64_t)st->num_cus * (bpc < per_cu ? bpc : per_cu);
+    return launch(f, (int)(need < cap ? need : cap), block, P, stream);
+  }
   if (use_stream) {
     // one workgroup per CU, fewer when there are fewer rows than waves
     const int64_t need = (num_tokens + block / 64 - 1) / (block / 64);
@@ -1425,7 +1454,7 @@ static int route_bwd_impl(const void* const* sources, int num_sources, int64_t n
     int bpc = 1;
     rc = get_bwd_rows(*st, rnch, num_sources, add ? kBwdRowsAdd : kBwdRowsPlain, &f, &bpc);
     if (rc != ATTNRES_OK) return rc;
-    return route_bwd_finish(f, bwd_rows_grid(num_tokens, st->num_cus, bpc), 64 * ATTNRES_BWD_ROWS_WAVES, 0, *st,
+    return route_bwd_finish(f, bwd_rows_grid(num_tokens, st->num_cus, bpc), 64 * ATTNRES_ROWS_WAVES, 0, *st,
                             nchunk, sources, num_sources, num_tokens, hidden, src_ld, query, gain, param_dtype, eps,
                             grad_out, grad_out_dtype, grad_out_ld, grad_lse, grad_sources, grad_ld, workspace,
                             workspace_bytes, grad_query, grad_gain, stream, addend);
@@ -1523,7 +1552,7 @@ int attnres_route_bwd_defer(const void* const* sources, int num_sources, int64_t
     int bpc = 1;
     rc = get_bwd_rows(*st, nch, num_sources, kBwdRowsDefer, &f, &bpc);
     if (rc != ATTNRES_OK) return rc;
-    return route_bwd_finish(f, bwd_rows_grid(num_tokens, st->num_cus, bpc), 64 * ATTNRES_BWD_ROWS_WAVES, 0, *st,
+    return route_bwd_finish(f, bwd_rows_grid(num_tokens, st->num_cus, bpc), 64 * ATTNRES_ROWS_WAVES, 0, *st,
                             hidden / 8, sources, num_sources, num_tokens, hidden, src_ld, query, gain, param_dtype,
                             eps, grad_out, grad_out_dtype, grad_out_ld, grad_lse, grads, grad_ld, workspace,
                             workspace_bytes, grad_query, grad_gain, stream, adds, coef, qfold);
@@ -1805,7 +1834,7 @@ int attnres_route_bwd_queries(const void* const* sources, int num_sources, int64
                 num_sources, mqg_lds, v);
   const int block = v == 1 ? round64(nchunk) : round64((nchunk + 1) / 2);
   const int rows_v = mqg ? mqg_rows_v(nchunk) : 0;
-  const int mqg_block = rows_v > 0 ? 64 * ATTNRES_BWD_ROWS_WAVES : round64((nchunk + 1) / 2);
+  const int mqg_block = rows_v > 0 ? 64 * ATTNRES_ROWS_WAVES : round64((nchunk + 1) / 2);
   hipFunction_t f = nullptr, fq = nullptr;
   int bpc = 1, bpcq = 1;
   if (rows_v > 0) {
@@ -1882,7 +1911,7 @@ int attnres_route_bwd_queries(const void* const* sources, int num_sources, int64
   int per_cu = mqg ? bpc : (bpc < 2 ? bpc : 2);
   if (tuning().bwd_per_cu > 0 && tuning().bwd_per_cu < per_cu) per_cu = tuning().bwd_per_cu;
   int64_t grid = (int64_t)st->num_cus * per_cu;
-  const int64_t units = rows_v > 0 ? (num_tokens + ATTNRES_BWD_ROWS_WAVES - 1) / ATTNRES_BWD_ROWS_WAVES : num_tokens;
+  const int64_t units = rows_v > 0 ? (num_tokens + ATTNRES_ROWS_WAVES - 1) / ATTNRES_ROWS_WAVES : num_tokens;
   if (grid > units) grid = units;
   rc = mqg ? launch(f, (int)grid, mqg_block, P, stream, 1, mqg_lds) : launch(f, (int)grid, block, P, stream);
   if (rc != ATTNRES_OK || !want_q) return rc;
@@ -1944,7 +1973,7 @@ int attnres_merge_bwd(const void* partial, int64_t num_tokens, int hidden, int p
   int64_t grid = 0;
   const int rnch = merge_bwd_rows_nch(pbf, ibf, hidden, num_tokens, st->num_cus);
   if (rnch > 0) {
-    block = 64 * ATTNRES_BWD_ROWS_WAVES;
+    block = 64 * ATTNRES_ROWS_WAVES;
     rc = get_merge_bwd_rows(*st, rnch, &f, &bpc);
     if (rc != ATTNRES_OK) return rc;
     grid = bwd_rows_grid(num_tokens, st->num_cus, bpc, rnch <= 4 ? 2 : 1);

@@ -1336,6 +1336,77 @@ __device__ __forceinline__ void merge_stream_body(const attnres_merge_params& P)
 }
 
 
+// The same merge for bf16 rows of up to 3 KiB of any width (NCH = the row's KiB,
+// rounded up), one wave per token row: a wave requests a token's partial and
+// inter rows together, through buffer resources of the row's bytes (chunks past
+// the row end read zeros, their stores are dropped); the query stays in
+// registers and nothing crosses waves.  Several workgroups per CU overlap one
+// wave's loads with another's arithmetic and stores, where one row in flight per
+// wave (merge_stream_body) or a workgroup per row leaves narrow rows waiting
+// (hidden 512, 32768 rows: 31.5 -> 17.2 us, 5.9 TB/s).
+template <int NCH>
+__device__ __forceinline__ void merge_rows_body(const attnres_merge_params& P) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float qw[NCH][8];
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int i = c * 64 + lane;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) qw[c][e] = 0.f;
+    if (i < P.nchunk) load_param<8>(P.query, (int64_t)i * 8, P.param_bf16, qw[c]);
+  }
+  const uint32_t n_tok = (uint32_t)P.n_tokens;
+  const uint32_t nw = gridDim.x * ATTNRES_ROWS_WAVES;
+  const uint32_t row_size = (uint32_t)P.d * 2;
+  const uint32_t lane_off = (uint32_t)lane * 16;
+  auto row_at = [&](const void* base, int64_t ld, uint32_t t) {
+    return row_rsrc(const_cast<char*>(uniform_ptr(reinterpret_cast<uint64_t>(base) + (uint64_t)t * ((uint64_t)ld * 2))),
+                    row_size);
+  };
+  auto lane63 = [](float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+  };
+  for (uint32_t t = blockIdx.x * ATTNRES_ROWS_WAVES + (uint32_t)wave; t < n_tok; t += nw) {
+    t = __builtin_amdgcn_readfirstlane(t);
+    u32x4 p[NCH], x[NCH];
+    const __amdgpu_buffer_rsrc_t pr = row_at(P.partial, P.partial_ld, t), ir = row_at(P.inter, P.inter_ld, t);
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) p[c] = ld_row_nt(pr, lane_off + (uint32_t)(c * 1024));
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) x[c] = ld_row_nt(ir, lane_off + (uint32_t)(c * 1024));
+    const float lse = ld_scalar_f32(P.inter_lse + t);
+    float ss = 0.f, dt = 0.f;
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        ss = dot2_bf16(p[c][w], p[c][w], ss);
+        dt = __builtin_fmaf(bf_lo(p[c][w]), qw[c][2 * w], dt);
+        dt = __builtin_fmaf(bf_hi(p[c][w]), qw[c][2 * w + 1], dt);
+      }
+    }
+    const float inv = __builtin_amdgcn_rsqf(lane63(wave_sum_to_lane63(ss)) * P.inv_d + P.eps);
+    const float logit = lane63(wave_sum_to_lane63(dt)) * inv;
+    const float pi = 1.0f / (1.0f + __expf(-(logit - lse)));
+    if (lane == 0) {
+      if (P.logit) P.logit[t] = logit;
+      if (P.inv_rms) P.inv_rms[t] = inv;
+    }
+    const __amdgpu_buffer_rsrc_t orr = row_at(P.out, P.out_ld, t);
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      u32x4 o;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float il = bf_lo(x[c][w]), ih = bf_hi(x[c][w]);
+        o[w] = pack_bf16(__builtin_fmaf(pi, bf_lo(p[c][w]) - il, il), __builtin_fmaf(pi, bf_hi(p[c][w]) - ih, ih));
+      }
+      st_row(orr, lane_off + (uint32_t)(c * 1024), o);
+    }
+  }
+}
+
 // ------------------------------------------------------ stream body --
 //
 // Prefill kernel: one wave64 owns one token row at a time, and the S source
@@ -2418,12 +2489,12 @@ template <int NCH>
 __device__ __forceinline__ void rows_query_partial(const float4* dq_lds, float* part, int d, int nchunk) {
   constexpr int ROW4 = NCH * 2 * 64;
   float4* prow = reinterpret_cast<float4*>(part + (int64_t)blockIdx.x * d);
-  for (int j = threadIdx.x; j < ROW4; j += 64 * ATTNRES_BWD_ROWS_WAVES) {
+  for (int j = threadIdx.x; j < ROW4; j += 64 * ATTNRES_ROWS_WAVES) {
     const int c = j >> 7, h = (j >> 6) & 1, l = j & 63;
     if (c * 64 + l >= nchunk) continue;
     float4 a = dq_lds[j];
 #pragma unroll
-    for (int w = 1; w < ATTNRES_BWD_ROWS_WAVES; ++w) {
+    for (int w = 1; w < ATTNRES_ROWS_WAVES; ++w) {
       const float4 b = dq_lds[w * ROW4 + j];
       a.x += b.x;
       a.y += b.y;
@@ -2463,8 +2534,8 @@ __device__ __forceinline__ void route_bwd_rows_body(const attnres_route_bwd_para
   constexpr int NP = 4 * H2;
   constexpr int SEG = S <= 8 ? 8 : 16;  // lanes of the softmax
   constexpr int ROW4 = NCH * 2 * 64;    // float4 slots of one query-gradient row
-  __shared__ float red[ATTNRES_BWD_ROWS_WAVES][NP];
-  __shared__ float4 dq_lds[ATTNRES_BWD_ROWS_WAVES * ROW4];
+  __shared__ float red[ATTNRES_ROWS_WAVES][NP];
+  __shared__ float4 dq_lds[ATTNRES_ROWS_WAVES * ROW4];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -2498,14 +2569,14 @@ __device__ __forceinline__ void route_bwd_rows_body(const attnres_route_bwd_para
 
   // 32-bit wave-uniform row counters (scalar loop control, as in stream_body)
   const uint32_t n_tok = (uint32_t)P.n_tokens;
-  const uint32_t nw = gridDim.x * ATTNRES_BWD_ROWS_WAVES;
+  const uint32_t nw = gridDim.x * ATTNRES_ROWS_WAVES;
   const uint32_t row_size = (uint32_t)P.d * 2;
   const uint32_t lane_off = (uint32_t)lane * 16;
   auto row_at = [&](const void* base, int64_t ld, uint32_t t) {
     return row_rsrc(const_cast<char*>(uniform_ptr(reinterpret_cast<uint64_t>(base) + (uint64_t)t * ((uint64_t)ld * 2))),
                     row_size);
   };
-  for (uint32_t t = blockIdx.x * ATTNRES_BWD_ROWS_WAVES + (uint32_t)wave; t < n_tok; t += nw) {
+  for (uint32_t t = blockIdx.x * ATTNRES_ROWS_WAVES + (uint32_t)wave; t < n_tok; t += nw) {
     t = __builtin_amdgcn_readfirstlane(t);
     // ---- the whole token in one go ----
     u32x4 x[S][NCH], g[NCH];
@@ -3157,7 +3228,7 @@ __device__ __forceinline__ void route_bwd_mqg_body(const attnres_route_bwd_mq_pa
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  constexpr int RW = ATTNRES_BWD_ROWS_WAVES;
+  constexpr int RW = ATTNRES_ROWS_WAVES;
   const int wave = ROWS ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
   const int block = ROWS ? 64 * RW : P.block;
   const int nwaves = (block + 63) >> 6;
@@ -3855,7 +3926,7 @@ __device__ __forceinline__ void merge_bwd_body(const attnres_merge_bwd_params& P
 template <int NCH>
 __device__ __forceinline__ void merge_bwd_rows_body(const attnres_merge_bwd_params& P) {
   constexpr int ROW4 = NCH * 2 * 64;  // float4 slots of one query-gradient row
-  __shared__ float4 dq_lds[ATTNRES_BWD_ROWS_WAVES * ROW4];
+  __shared__ float4 dq_lds[ATTNRES_ROWS_WAVES * ROW4];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -3868,7 +3939,7 @@ __device__ __forceinline__ void merge_bwd_rows_body(const attnres_merge_bwd_para
     if (i < P.nchunk) load_param<8>(P.query, (int64_t)i * 8, P.param_bf16, qw[c]);
   }
   const uint32_t n_tok = (uint32_t)P.n_tokens;
-  const uint32_t nw = gridDim.x * ATTNRES_BWD_ROWS_WAVES;
+  const uint32_t nw = gridDim.x * ATTNRES_ROWS_WAVES;
   const uint32_t row_size = (uint32_t)P.d * 2;
   const uint32_t lane_off = (uint32_t)lane * 16;
   auto row_at = [&](const void* base, uint32_t t) {
@@ -3877,7 +3948,7 @@ __device__ __forceinline__ void merge_bwd_rows_body(const attnres_merge_bwd_para
   auto lane63 = [](float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
   };
-  for (uint32_t t = blockIdx.x * ATTNRES_BWD_ROWS_WAVES + (uint32_t)wave; t < n_tok; t += nw) {
+  for (uint32_t t = blockIdx.x * ATTNRES_ROWS_WAVES + (uint32_t)wave; t < n_tok; t += nw) {
     t = __builtin_amdgcn_readfirstlane(t);
     u32x4 p[NCH], x[NCH], g[NCH];
     const __amdgpu_buffer_rsrc_t pr = row_at(P.partial, t), ir = row_at(P.inter, t), gr = row_at(P.grad_out, t);
@@ -4225,6 +4296,12 @@ MERGE_V(2)
   extern "C" __global__ void __launch_bounds__(256) attnres_merge_stream_fm_c##NCH(attnres_merge_params P) { \
     merge_stream_body<NCH, false>(P);                                                                \
   }
+#define MERGE_ROWS(NCH)                                                                              \
+  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_ROWS_WAVES) attnres_merge_rows_c##NCH(   \
+      attnres_merge_params P) {                                                                      \
+    merge_rows_body<NCH>(P);                                                                         \
+  }
+MERGE_ROWS(1) MERGE_ROWS(2) MERGE_ROWS(3)
 MERGE_STREAM(1)
 MERGE_STREAM(2)
 MERGE_STREAM(3)
@@ -4410,7 +4487,7 @@ BWD_DQW(bf, true, 1) BWD_DQW(bf, true, 2) BWD_DQW(f32, false, 1) BWD_DQW(f32, fa
     route_bwd_mqg_body<S, 2, NQ4>(P);                                                           \
   }
 #define BWD_MQG_ROWS_ONE(S, V, NQ4)                                                             \
-  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_BWD_ROWS_WAVES)                     \
+  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_ROWS_WAVES)                     \
       __attribute__((amdgpu_waves_per_eu(MQG_ROWS_EU(S, V, NQ4))))                              \
       attnres_route_bwd_mqg_rows_v##V##_s##S##_q##NQ4(attnres_route_bwd_mq_params P) {          \
     route_bwd_mqg_body<S, V, NQ4, true>(P);                                                     \
@@ -4514,25 +4591,25 @@ BWD_STREAM_ONE_DEFER(8, 8, 2) BWD_STREAM_ONE_DEFER(9, 8, 3)
 #define BWD_ROWS_EU(S, NCH, R) \
   (4 * (NCH) * (R) + 16 * (NCH) + 40 <= 128 ? 4 : 4 * (NCH) * (R) + 16 * (NCH) + 40 <= 168 ? 3 : 2)
 #define BWD_ROWS_ONE(S, NCH)                                                                             \
-  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_BWD_ROWS_WAVES)                              \
+  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_ROWS_WAVES)                              \
       __attribute__((amdgpu_waves_per_eu(BWD_ROWS_EU(S, NCH, (S) + 1))))                                 \
       attnres_route_bwd_rows_c##NCH##_s##S(attnres_route_bwd_params P) {                                 \
     route_bwd_rows_body<S, NCH>(P);                                                                      \
   }
 #define BWD_ROWS_ADD(S, NCH)                                                                             \
-  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_BWD_ROWS_WAVES)                              \
+  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_ROWS_WAVES)                              \
       __attribute__((amdgpu_waves_per_eu(BWD_ROWS_EU(S, NCH, 2 * (S) + 1))))                             \
       attnres_route_bwd_rows_c##NCH##_s##S##_add(attnres_route_bwd_params P) {                           \
     route_bwd_rows_body<S, NCH, true>(P);                                                                \
   }
 #define BWD_ROWS_DEFER(S, NCH)                                                                           \
-  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_BWD_ROWS_WAVES)                              \
+  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_ROWS_WAVES)                              \
       __attribute__((amdgpu_waves_per_eu(BWD_ROWS_EU(S, NCH, (S) + 2))))                                 \
       attnres_route_bwd_rows_c##NCH##_s##S##_defer(attnres_route_bwd_params P) {                         \
     route_bwd_rows_body<S, NCH, true, true>(P);                                                          \
   }
 #define MERGE_BWD_ROWS(NCH)                                                                              \
-  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_BWD_ROWS_WAVES)                              \
+  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_ROWS_WAVES)                              \
       __attribute__((amdgpu_waves_per_eu(BWD_ROWS_EU(0, NCH, 3))))                                       \
       attnres_merge_bwd_rows_c##NCH(attnres_merge_bwd_params P) {                                        \
     merge_bwd_rows_body<NCH>(P);                                                                         \

@@ -14,7 +14,7 @@
 
 #define ATTNRES_KMAX_SOURCES 16   /* S templates instantiated: 0..16 */
 #define ATTNRES_KMAX_WAVES 8      /* 512 threads per workgroup */
-#define ATTNRES_BWD_ROWS_WAVES 4  /* waves (token rows) per workgroup of the narrow rows' backward */
+#define ATTNRES_ROWS_WAVES 4  /* waves (token rows) per workgroup of the narrow rows' kernels */
 
 /* How the last source slot (the partial block) is formed before routing. */
 #define ATTNRES_MODE_PLAIN 0      /* partial is read as-is */

@@ -2,6 +2,7 @@
 row widths, source counts and row counts where they can go wrong: one chunk
 less and more than a whole KiB, the narrowest row, waves without a row."""
 
+import numpy as np
 import pytest
 import torch
 
@@ -11,6 +12,7 @@ from oracle import attnres_oracle as O
 
 from .test_gpu_accumulate import _call, _case
 from .test_gpu_backward import Norm, _bwd_kernel_name, bwd_queries_kernel, check_grad, make_case, np64, oracle_grads
+from .test_gpu_parity import check_bf16, merge_kernel
 
 pytestmark = pytest.mark.gpu
 
@@ -140,3 +142,24 @@ def test_row_per_wave_batched_backward_matches_oracle(gpu, D, S, N, Q):
         dx = dx + b["dx"]
         check_grad(qs.grad[j], b["dqw"], torch.bfloat16, f"dquery[{j}]")
     check_grad(buf.grad.reshape(S, N, D), dx, torch.bfloat16, "dsources")
+
+
+FORWARD_MERGE_CASES = [(8, 1024, None), (504, 1025, None), (520, 3001, torch.float32), (1536, 1030, None)]
+
+
+@pytest.mark.parametrize("D,N,qd", FORWARD_MERGE_CASES,
+                         ids=[f"D{c[0]}-N{c[1]}{'-qf32' if c[2] else ''}" for c in FORWARD_MERGE_CASES])
+def test_narrow_merge_matches_oracle(gpu, D, N, qd):
+    print(f"narrow merge D={D} N={N} query={qd}", flush=True)
+    assert merge_kernel(N, D, qd or torch.bfloat16) == f"attnres_merge_rows_c{(D + 511) // 512}"
+    g = torch.Generator(device="cpu").manual_seed(D + N)
+    p = (torch.randn(N, D, generator=g) * 2).to(torch.bfloat16).to(gpu)
+    inter = torch.randn(N, D, generator=g).to(torch.bfloat16).to(gpu)
+    q = (torch.randn(D, generator=g) * 0.1).to(qd or torch.bfloat16).to(gpu)
+    lse = torch.randn(N, generator=g).to(gpu)
+    with torch.no_grad():
+        out, logit, inv = ops.merge(p, q, inter, lse, 1e-5)
+    ref = O.merge(np64(p), np64(q), np64(inter), np64(lse), 1e-5)
+    check_bf16(out, ref["out"], f"narrow merge D={D} N={N}")
+    np.testing.assert_allclose(np64(logit), ref["logit"], rtol=1e-4, atol=1e-4)
+    np.testing.assert_allclose(np64(inv), ref["inv_rms"], rtol=1e-5)
