@@ -20,6 +20,7 @@ Run ``python -m kotodama_amd.build`` or call :func:`build`.
 
 from __future__ import annotations
 
+import importlib.util
 import os
 import subprocess
 import sys
@@ -79,9 +80,12 @@ def build(verbose: bool = False, out_dir: Path | None = None, defines: tuple = (
     extra = [f"-D{d}" for d in defines]
     with tempfile.TemporaryDirectory(prefix="attnres_build_", dir=libdir) as tmp:
         tmpd = Path(tmp)
+        procs = []
         native_o = tmpd / "attnres_torch.o"
-        native = _native_cmd(native_o)
-        procs = [(native, subprocess.Popen(native, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True))]
+        with_torch = importlib.util.find_spec("torch") is not None  # the C-ABI library needs no torch
+        if with_torch:
+            native = _native_cmd(native_o)
+            procs.append((native, subprocess.Popen(native, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)))
         for part in range(NUM_PARTS):
             out = tmpd / f"attnres_gfx950_part{part}.hsaco"
             cmd = [hipcc, *HIP_FLAGS, *extra, f"-DATTNRES_PART={part}", f"-I{CSRC}", str(CSRC / "attnres_kernels.hip"),
@@ -125,16 +129,17 @@ def build(verbose: bool = False, out_dir: Path | None = None, defines: tuple = (
                 str(so_tmp),
             ]
         )
-        import torch
-
-        torch_lib = Path(torch.__file__).parent / "lib"
-        native_tmp = tmpd / NATIVE_NAME
-        _run(["g++", "-shared", str(native_o), f"-L{tmpd}", "-lattnres_hip", f"-L{torch_lib}", "-ltorch_python",
-              "-ltorch_cpu", "-ltorch_hip", "-lc10_hip", "-lc10", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{torch_lib}",
-              "-o", str(native_tmp)])
         final = libdir / LIB_NAME
         os.replace(so_tmp, final)  # atomic: a reader never sees a half-written library
-        os.replace(native_tmp, libdir / NATIVE_NAME)
+        if with_torch:
+            import torch
+
+            torch_lib = Path(torch.__file__).parent / "lib"
+            native_tmp = tmpd / NATIVE_NAME
+            _run(["g++", "-shared", str(native_o), f"-L{libdir}", "-lattnres_hip", f"-L{torch_lib}", "-ltorch_python",
+                  "-ltorch_cpu", "-ltorch_hip", "-lc10_hip", "-lc10", "-Wl,-rpath,$ORIGIN",
+                  f"-Wl,-rpath,{torch_lib}", "-o", str(native_tmp)])
+            os.replace(native_tmp, libdir / NATIVE_NAME)
     if verbose:
         print(f"built {final}", flush=True)
     return final
