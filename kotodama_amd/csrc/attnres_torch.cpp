@@ -478,6 +478,11 @@ bool take(PyObject* o, int64_t* v) {
   }
   return true;
 }
+// exactly True or False (another truthy value is left to Python)
+bool take(PyObject* o, bool* v) {
+  *v = o == Py_True;
+  return PyBool_Check(o);
+}
 // out_dtype: a torch.dtype, or None for the promotion of the sources' and the parameters' dtypes
 bool take_dtype(PyObject* o, const Tensor& src, const Tensor& query, const Tensor& gain, at::ScalarType* t) {
   if (THPDtype_Check(o)) {
@@ -547,11 +552,13 @@ PyObject* pack(const Routed& r, int64_t form) {
 PyObject* py_route(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Tensor buf, query, gain;
+  bool ww, wl, wa;
   int64_t num = 0, form = 0;
   double eps = 0;
   at::ScalarType dt;
   if (n != 11 || !take(a[0], false, &buf) || !take(a[1], &num) || !take(a[2], false, &query) ||
-      !take(a[3], true, &gain) || !take(a[4], &eps) || !take_dtype(a[5], buf, query, gain, &dt) || !take(a[9], &form) || !unwatched())
+      !take(a[3], true, &gain) || !take(a[4], &eps) || !take_dtype(a[5], buf, query, gain, &dt) || !take(a[6], &ww) || !take(a[7], &wl) || !take(a[8], &wa) ||
+      !take(a[9], &form) || !unwatched())
     return none();
   const bool rec = recorded({&buf, &query, &gain});
   if (rec && (a[10] == Py_None || num < 1 || !no_tangent(buf) || !no_tangent(query) || !no_tangent(gain)))
@@ -559,8 +566,7 @@ PyObject* py_route(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Routed r;
   {
     pybind11::gil_scoped_release nogil;
-    if (!route_rows(Sources::stacked(buf, num), query, gain, eps, dt, a[6] == Py_True, a[7] == Py_True,
-                    a[8] == Py_True, form == kRows, &r))
+    if (!route_rows(Sources::stacked(buf, num), query, gain, eps, dt, ww, wl, wa, form == kRows, &r))
       r.out = Tensor();
   }
   if (!r.out.defined()) return none();
@@ -581,13 +587,14 @@ PyObject* py_route_list(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   std::vector<Tensor> srcs;
   Tensor query, gain;
+  bool ww, wl, wa;
   double eps = 0;
   int64_t form = 0;
   at::ScalarType dt;
   if (n != 10 || !take_list(a[0], &srcs) || srcs.empty() || !take(a[1], false, &query) || !take(a[2], true, &gain) ||
-      !take(a[3], &eps) || !take_dtype(a[4], srcs[0], query, gain, &dt) || !take(a[8], &form) || !unwatched())
+      !take(a[3], &eps) || !take_dtype(a[4], srcs[0], query, gain, &dt) || !take(a[5], &ww) || !take(a[6], &wl) ||
+      !take(a[7], &wa) || !take(a[8], &form) || !unwatched())
     return none();
-  const bool ww = a[5] == Py_True, wa = a[7] == Py_True;
   const bool rec = recorded(srcs) || recorded({&query, &gain});
   if (rec) {
     if (a[9] != Py_True || ww || wa || !no_tangent(query) || !no_tangent(gain)) return none();
@@ -597,7 +604,7 @@ PyObject* py_route_list(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Routed r;
   {
     pybind11::gil_scoped_release nogil;
-    if (!route_rows(Sources::list(srcs), query, gain, eps, dt, ww, a[6] == Py_True, wa, form == kRows, &r)) r.out = Tensor();
+    if (!route_rows(Sources::list(srcs), query, gain, eps, dt, ww, wl, wa, form == kRows, &r)) r.out = Tensor();
   }
   if (!r.out.defined()) return none();
   if (rec) {
@@ -636,11 +643,11 @@ PyObject* py_block_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor arena, delta, query, gain;
   int64_t nc = 0;
   double eps = 0;
-  if (n != 8 || !take(a[0], false, &arena) || !take(a[1], &nc) || !PyBool_Check(a[2]) || !take(a[3], true, &delta) ||
-      !take(a[4], false, &query) || !take(a[5], true, &gain) || !take(a[6], &eps) || !unwatched() ||
+  bool commit, ww;
+  if (n != 8 || !take(a[0], false, &arena) || !take(a[1], &nc) || !take(a[2], &commit) || !take(a[3], true, &delta) ||
+      !take(a[4], false, &query) || !take(a[5], true, &gain) || !take(a[6], &eps) || !take(a[7], &ww) || !unwatched() ||
       recorded({&arena, &delta, &query, &gain}))
     return none();
-  const bool commit = a[2] == Py_True, ww = a[7] == Py_True;
   const int64_t s = nc + (commit ? 1 : 0) + 1;
   const Sources src = Sources::stacked(arena, std::min<int64_t>(s, arena.dim() > 0 ? arena.size(0) : 0));
   if (!src.ok || s < 1 || s > arena.size(0) || query.dim() != 1) return none();

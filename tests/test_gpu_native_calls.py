@@ -120,6 +120,11 @@ def test_calls_left_to_the_ops(gpu):
     assert not taken(buf.requires_grad_())  # recorded, and the caller did not ask for that
     with torch.no_grad():
         assert taken(buf)
+    # a flag that is true but not True is not read as False
+    with torch.no_grad():
+        assert native.route(buf, 2, query, gain, 1e-5, BF, 1, 1, False, ops._TUPLE, None) is None
+        assert ops.route_call(buf, 2, query, gain, 1e-5, BF, want_weights=1)[1].shape == (1, 2, 2, 9)
+        assert ops.block_step_call(buf.clone(), 1, 0, None, query, gain, 1e-5, 1)[1].shape == (2, 2, 9)
     # ... and the drop-in's result for them is the op's
     with torch.no_grad():
         strided = buf.transpose(1, 2)
