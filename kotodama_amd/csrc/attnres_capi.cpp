@@ -61,6 +61,7 @@ int hip_fail(hipError_t e, const char* what) {
 // Route kernel variants: type combo x S x V x (single/multi query).
 enum TypeCombo { kBfDot2 = 0, kBfFma = 1, kF32Fma = 2, kTypeCombos = 3 };
 constexpr int kNumS = ATTNRES_KMAX_SOURCES + 1;
+constexpr int kRouteRowsMaxS = 9;  // sources of the narrow rows' routing kernel
 constexpr int kRouteFuncs = kTypeCombos * kNumS * 2 * 2;
 constexpr int kMergeFuncs = 4 * 2;
 constexpr int kStreamMaxChunks = 8;  // rows of up to 8 KiB
@@ -104,6 +105,7 @@ struct DeviceState {
   KernelSlot route_qg[kNumS * 2];  // batched-query kernels: S x V
   KernelSlot stream[kStreamFuncs];
   KernelSlot merge[kMergeFuncs];
+  KernelSlot route_rows[kRouteRowsMaxS + 1];  // row-per-wave routing of narrow rows: S (2..9)
   KernelSlot merge_rows[3];  // row-per-wave merge of narrow rows: row KiB (1..3)
   KernelSlot merge_stream[2 * kStreamMaxChunks];  // row-per-wave merge: query path x row KiB
   KernelSlot bwd[kBwdFuncs];
@@ -343,6 +345,13 @@ int get_route(DeviceState& st, int combo, int s, int v, bool multiq, int block, 
   char name[96];
   snprintf(name, sizeof(name), "attnres_route_%s_s%d_v%d_%s", combo_names[combo], s, v, multiq ? "qn" : "q1");
   return slot_get(st, st.route[route_index(combo, s, v, multiq)], part_of_route(s), name, block, 0, f, bpc);
+}
+
+// The narrow rows' routing kernel (rows of up to 3 KiB).
+int get_route_rows(DeviceState& st, int s, hipFunction_t* f, int* bpc) {
+  char name[96];
+  snprintf(name, sizeof(name), "attnres_route_rows_c3_s%d", s);
+  return slot_get(st, st.route_rows[s], 11, name, 64 * ATTNRES_ROWS_WAVES, 0, f, bpc);
 }
 
 // Batched-query kernel (bf16 sources and parameters, Q >= 2) with `lds` bytes
@@ -678,6 +687,7 @@ int launch(hipFunction_t f, int grid, int block, Params& P, void* stream, int gr
 // kernel with V chunks per thread.
 struct RouteChoice {
   bool stream = false;
+  bool rows = false;  // the narrow rows' kernel
   int combo = 0;
   int nch = 0;    // streaming: KiB per row
   int variant = kStreamPlain;  // streaming: plain / pointer table / fused
@@ -752,6 +762,25 @@ RouteChoice choose_route(int num_sources, int64_t num_tokens, int hidden, int sr
   return ch;
 }
 
+// Whether a call goes to the narrow rows' routing kernel: plain bf16 calls of
+// one query, 2 to 9 sources and rows of more than 2 and up to 3 KiB, from four
+// rows per CU on.  Against the kernel before (us per call, S = 3 / 5 / 9):
+// hidden 1536 at 1500 rows 7.5 / 9.2 / 12.1 -> 6.8 / 8.2 / 11.5, at 8192
+// 24.5 / 34.8 / 55.4 -> 18.6 / 27.4 / 44.8, at 32768 81 / 122 / 204 -> 64 / 98 /
+// 169 (6.2 TB/s at S = 5); hidden 1032 at 8192 rows 16.5 / 23.1 / 40.0 -> 14.5 /
+// 21.2 / 35.4; hidden 1280, 5 sources, 23.8 -> 23.5 at 8192 and 90.4 -> 81.3 at
+// 32768.  One source is up to 5% slower (hidden 1536, 4096 rows 7.1 -> 7.5), and
+// rows of 2 KiB and less go either way (hidden 1024 at 8192 rows: 3 sources 14.7
+// -> 13.5, 9 sources 30.6 -> 33.0; hidden 64, 5 sources 7.1 -> 7.7).
+bool route_rows_shape(int num_sources, int64_t num_tokens, int hidden, int src_dtype, int param_dtype, int out_dtype,
+                      int num_queries, int mode, int num_cus) {
+  return src_dtype == ATTNRES_DTYPE_BF16 && param_dtype == ATTNRES_DTYPE_BF16 && out_dtype == ATTNRES_DTYPE_BF16 &&
+         num_queries == 1 && mode == ATTNRES_MODE_PLAIN && num_sources >= 2 && num_sources <= kRouteRowsMaxS &&
+         hidden > 1024 && hidden <= 1536 && hidden % 8 == 0 && num_tokens >= 4LL * num_cus &&
+         num_tokens < (int64_t)1 << 31 && g_policy.load(std::memory_order_relaxed) == ATTNRES_POLICY_AUTO &&
+         tuning().stream < 0;
+}
+
 // The whole kernel choice of one routing call (family, streaming variant,
 // chunks per thread, batched-query kernel), shared by the launch and the
 // kernel-name query.  The streaming kernel addresses equally spaced sources
@@ -761,6 +790,14 @@ RouteChoice choose_route(int num_sources, int64_t num_tokens, int hidden, int sr
 // workgroup kernel).
 RouteChoice plan_route(int num_sources, int64_t num_tokens, int hidden, int src_dtype, int param_dtype,
                        int out_dtype, int num_queries, int mode, bool equally_spaced, const DeviceState& st) {
+  if (route_rows_shape(num_sources, num_tokens, hidden, src_dtype, param_dtype, out_dtype, num_queries, mode,
+                       st.num_cus)) {
+    RouteChoice ch;
+    ch.rows = true;
+    ch.combo = kBfDot2;
+    ch.block = 64 * ATTNRES_ROWS_WAVES;
+    return ch;
+  }
   const bool stream_ok = !(mode == ATTNRES_MODE_ACCUM && num_sources < 2);
   RouteChoice ch = choose_route(num_sources, num_tokens, hidden, src_dtype, param_dtype, num_queries, st.num_cus,
                                 stream_ok, mode != ATTNRES_MODE_PLAIN);
@@ -777,7 +814,9 @@ RouteChoice plan_route(int num_sources, int64_t num_tokens, int hidden, int src_
 
 void kernel_name_of(const RouteChoice& ch, int num_sources, int num_queries, bool out_bf, char* buf, size_t n) {
   static const char* combo_names[kTypeCombos] = {"bf_d2", "bf_fm", "f32_fm"};
-  if (ch.stream) {
+  if (ch.rows) {
+    snprintf(buf, n, "attnres_route_rows_c3_s%d", num_sources);
+  } else if (ch.stream) {
     snprintf(buf, n, "attnres_stream_%s_o%s_c%d_%s", combo_names[ch.combo], out_bf ? "bf" : "f32", ch.nch,
              kStreamVariantNames[ch.variant]);
   } else {
@@ -904,7 +943,8 @@ int route_launch(const void* const* sources, int num_sources, int64_t num_tokens
   }
   const RouteChoice ch = plan_route(num_sources, num_tokens, hidden, src_dtype, param_dtype, out_dtype, num_queries,
                                     mode, equally_spaced, *st);
-  if (!ch.stream && ch.v == 0) return fail(ATTNRES_ERR_UNSUPPORTED, "hidden=%d has no launch shape", hidden);
+  if (!ch.rows && !ch.stream && ch.v == 0)
+    return fail(ATTNRES_ERR_UNSUPPORTED, "hidden=%d has no launch shape", hidden);
 
   hipFunction_t f = nullptr;
   int bpc = 1;
@@ -925,6 +965,16 @@ int route_launch(const void* const* sources, int num_sources, int64_t num_tokens
                     ? 1
                     : stream_out_batch(num_sources, out_row_bytes, slds, st->max_lds, waves);
     if (out_batch > 1) stream_lds = (size_t)waves * out_batch * out_row_bytes;
+  } else if (ch.rows) {
+    rc = get_route_rows(*st, num_sources, &f, &bpc);
+    if (rc != ATTNRES_OK) return rc;
+    // Two workgroups per CU keep enough rows in flight; with long row loops over
+    // five sources or more, one does (hidden 1536, 5 sources, one against two:
+    // 65536 rows 196 against 204 us, 16384 rows 51.7 against 52.6, but 8192 rows
+    // 28.2 against 27.2; 2 sources of hidden 1280 at 32768 rows 47.6 against 39.9).
+    const int per_cu = num_sources >= 5 && num_tokens >= 64LL * st->num_cus ? 1 : 2;
+    if (bpc > per_cu) bpc = per_cu;
+    work_units = (num_tokens + ATTNRES_ROWS_WAVES - 1) / ATTNRES_ROWS_WAVES;
   } else if (ch.qg_lds > 0) {
     rc = get_route_qg(*st, num_sources, ch.v, block, ch.qg_lds, &f, &bpc);
     if (rc != ATTNRES_OK) return rc;
@@ -1054,7 +1104,8 @@ int attnres_route_kernel_name(int num_sources, int64_t num_tokens, int hidden, i
   const int mode = fused == 0 ? ATTNRES_MODE_PLAIN : fused == 1 ? ATTNRES_MODE_ACCUM : ATTNRES_MODE_SET;
   const RouteChoice ch = plan_route(num_sources, num_tokens, hidden, src_dtype, param_dtype, out_dtype, num_queries,
                                     mode, equally_spaced != 0, *st);
-  if (!ch.stream && ch.v == 0) return fail(ATTNRES_ERR_UNSUPPORTED, "hidden=%d has no launch shape", hidden);
+  if (!ch.rows && !ch.stream && ch.v == 0)
+    return fail(ATTNRES_ERR_UNSUPPORTED, "hidden=%d has no launch shape", hidden);
   kernel_name_of(ch, num_sources, num_queries, out_dtype == ATTNRES_DTYPE_BF16, buf, (size_t)buf_len);
   return ATTNRES_OK;
 }

@@ -766,6 +766,114 @@ __device__ __forceinline__ void route_body(const attnres_route_params& P) {
   }
 }
 
+// ---------------------------------- row-per-wave routing of narrow rows --
+//
+// One query over bf16 rows of any width up to NCH KiB (3, the only one launched),
+// bf16 parameters and output: one wave per token row, every source row requested
+// at once through buffer resources of the row's bytes (chunks past the row end
+// read zeros, their stores are dropped), the 2S sums reduced by the transposing
+// tree through the wave's own LDS row, the softmax with lane s for source s, no
+// barrier.  Bound by memory: the streaming kernel's chain of one source row after
+// another in a single workgroup per CU, and the workgroup kernel's barriers, left
+// rows of this size waiting (hidden 1536, 5 sources, 32768 rows: 122 -> 98 us,
+// 6.2 TB/s).
+template <int S, int NCH>
+__device__ __forceinline__ void route_rows_body(const attnres_route_params& P) {
+  constexpr int NV = 2 * S;
+  constexpr int H2 = (NV + 3) / 4;
+  constexpr int NP = 4 * H2;
+  constexpr int SEG = S <= 8 ? 8 : 16;
+  __shared__ float red[ATTNRES_ROWS_WAVES][NP];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  u32x4 qw[NCH];  // packed folded query (bf16-exact)
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int i = c * 64 + lane;
+    qw[c] = u32x4{0, 0, 0, 0};
+    if (i < P.nchunk) {
+      float t[8];
+      load_qw<8>(P, 0, i, t);
+      qw[c] = u32x4{pack_bf16(t[0], t[1]), pack_bf16(t[2], t[3]), pack_bf16(t[4], t[5]), pack_bf16(t[6], t[7])};
+    }
+  }
+  const uint32_t n_tok = (uint32_t)P.n_tokens;
+  const uint32_t nw = gridDim.x * ATTNRES_ROWS_WAVES;
+  const uint32_t row_size = (uint32_t)P.d * 2;
+  const uint32_t lane_off = (uint32_t)lane * 16;
+  auto row_at = [&](const void* base, int64_t ld, uint32_t t) {
+    return row_rsrc(const_cast<char*>(uniform_ptr(reinterpret_cast<uint64_t>(base) + (uint64_t)t * ((uint64_t)ld * 2))),
+                    row_size);
+  };
+  for (uint32_t t = blockIdx.x * ATTNRES_ROWS_WAVES + (uint32_t)wave; t < n_tok; t += nw) {
+    t = __builtin_amdgcn_readfirstlane(t);
+    u32x4 x[S][NCH];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const __amdgpu_buffer_rsrc_t sr = row_at(P.src[s], P.src_ld, t);
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) x[s][c] = ld_row_nt(sr, lane_off + (uint32_t)(c * 1024));
+    }
+    float part[NP];
+#pragma unroll
+    for (int j = 0; j < NP; ++j) part[j] = 0.f;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          part[s] = dot2_bf16(x[s][c][w], x[s][c][w], part[s]);
+          part[S + s] = dot2_bf16(x[s][c][w], qw[c][w], part[S + s]);
+        }
+      }
+    }
+    wave_reduce_to_lds<H2>(part, red[wave], lane);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int ls = lane % SEG;
+    const bool slot = ls < S;
+    const float t_ss = slot ? red[wave][ls] : 0.f;
+    const float t_dot = slot ? red[wave][S + ls] : 0.f;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const float inv = __builtin_amdgcn_rsqf(t_ss * P.inv_d + P.eps);
+    const float logit = slot ? t_dot * inv : -__builtin_inff();
+    const float m = seg_max<SEG>(logit);
+    const float el = slot ? __expf(logit - m) : 0.f;
+    const float sum = seg_sum<SEG>(el);
+    const float wl = el * (1.0f / sum);
+    if (lane < S) {
+      if (P.weights) P.weights[(int64_t)lane * P.n_tokens + t] = wl;
+      if (P.logits) P.logits[(int64_t)t * S + lane] = logit;
+      if (P.inv_rms) P.inv_rms[(int64_t)t * S + lane] = inv;
+      if (lane == 0 && P.lse) P.lse[t] = m + __logf(sum);
+    }
+    float wgt[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      wgt[s] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wl), s));
+    const __amdgpu_buffer_rsrc_t orr = row_at(P.out, P.out_ld, t);
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+#pragma unroll
+      for (int s = 0; s < S; ++s) asm volatile("" : "+v"(x[s][c]));
+      u32x4 o;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        float lo = wgt[0] * bf_lo(x[0][c][w]), hi = wgt[0] * bf_hi(x[0][c][w]);
+#pragma unroll
+        for (int s = 1; s < S; ++s) {
+          lo = __builtin_fmaf(wgt[s], bf_lo(x[s][c][w]), lo);
+          hi = __builtin_fmaf(wgt[s], bf_hi(x[s][c][w]), hi);
+        }
+        o[w] = pack_bf16(lo, hi);
+      }
+      st_row(orr, lane_off + (uint32_t)(c * 1024), o);
+    }
+  }
+}
+
 // ------------------------------------------------- batched-query body --
 //
 // Phase-1 batching for bf16 sources and bf16 parameters (the serving
@@ -4614,12 +4722,19 @@ BWD_STREAM_ONE_DEFER(8, 8, 2) BWD_STREAM_ONE_DEFER(9, 8, 3)
       attnres_merge_bwd_rows_c##NCH(attnres_merge_bwd_params P) {                                        \
     merge_bwd_rows_body<NCH>(P);                                                                         \
   }
+#define ROUTE_ROWS(S, NCH)                                                                               \
+  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_ROWS_WAVES)                                  \
+      attnres_route_rows_c##NCH##_s##S(attnres_route_params P) {                                         \
+    route_rows_body<S, NCH>(P);                                                                          \
+  }
 #define BWD_ROWS_S(S) \
   BWD_ROWS_ONE(S, 1) BWD_ROWS_ONE(S, 2) BWD_ROWS_ONE(S, 3) BWD_ROWS_ADD(S, 1) BWD_ROWS_ADD(S, 2)
 #if ATTNRES_PART == 11 || defined(ATTNRES_ALL_PARTS)
 BWD_ROWS_S(1) BWD_ROWS_S(2) BWD_ROWS_S(3) BWD_ROWS_S(4) BWD_ROWS_S(5)
 BWD_ROWS_S(6) BWD_ROWS_S(7) BWD_ROWS_S(8) BWD_ROWS_S(9)
 BWD_ROWS_ADD(1, 3) BWD_ROWS_ADD(2, 3) BWD_ROWS_ADD(3, 3) BWD_ROWS_ADD(4, 3) BWD_ROWS_ADD(5, 3) BWD_ROWS_ADD(6, 3)
+ROUTE_ROWS(2, 3) ROUTE_ROWS(3, 3) ROUTE_ROWS(4, 3) ROUTE_ROWS(5, 3)
+ROUTE_ROWS(6, 3) ROUTE_ROWS(7, 3) ROUTE_ROWS(8, 3) ROUTE_ROWS(9, 3)
 MERGE_BWD_ROWS(1) MERGE_BWD_ROWS(2) MERGE_BWD_ROWS(3) MERGE_BWD_ROWS(4) MERGE_BWD_ROWS(5) MERGE_BWD_ROWS(6)
 BWD_ROWS_DEFER(2, 1) BWD_ROWS_DEFER(3, 1) BWD_ROWS_DEFER(4, 1) BWD_ROWS_DEFER(5, 1)
 BWD_ROWS_DEFER(6, 1) BWD_ROWS_DEFER(7, 1) BWD_ROWS_DEFER(8, 1)

@@ -2,6 +2,8 @@
 row widths, source counts and row counts where they can go wrong: one chunk
 less and more than a whole KiB, the narrowest row, waves without a row."""
 
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -12,7 +14,7 @@ from oracle import attnres_oracle as O
 
 from .test_gpu_accumulate import _call, _case
 from .test_gpu_backward import Norm, _bwd_kernel_name, bwd_queries_kernel, check_grad, make_case, np64, oracle_grads
-from .test_gpu_parity import check_bf16, merge_kernel
+from .test_gpu_parity import check_bf16, check_weights, merge_kernel, route_kernel
 
 pytestmark = pytest.mark.gpu
 
@@ -163,3 +165,81 @@ def test_narrow_merge_matches_oracle(gpu, D, N, qd):
     check_bf16(out, ref["out"], f"narrow merge D={D} N={N}")
     np.testing.assert_allclose(np64(logit), ref["logit"], rtol=1e-4, atol=1e-4)
     np.testing.assert_allclose(np64(inv), ref["inv_rms"], rtol=1e-5)
+
+
+def test_narrow_routing_policy(gpu):
+    cus = torch.cuda.get_device_properties(gpu).multi_processor_count
+    assert route_kernel(2, 4 * cus, 1032, 1) == "attnres_route_rows_c3_s2"
+    assert route_kernel(9, 8192, 1536, 1) == "attnres_route_rows_c3_s9"
+    for s, n, d, q in ((2, 4 * cus - 1, 1536, 1), (1, 8192, 1536, 1), (10, 8192, 1536, 1), (5, 8192, 1024, 1),
+                       (5, 8192, 1544, 1), (5, 8192, 1536, 2)):
+        assert "_rows_" not in route_kernel(s, n, d, q), (s, n, d, q)
+    prev = _capi.set_kernel_policy(_capi.POLICY_STREAM)
+    try:
+        assert "_rows_" not in route_kernel(5, 8192, 1536, 1)
+    finally:
+        _capi.set_kernel_policy(prev)
+
+
+# (hidden, sources, rows, separate allocations, gain): the narrowest and the widest row, a third
+# chunk of one lane, half and all lanes, the fewest rows, waves without a row, one and two
+# workgroups per CU (from 64 rows per CU on one, with 5 sources and more)
+ROUTE_CASES = [(1032, 2, 1024, False, True), (1032, 9, 16391, False, False), (1280, 5, 1027, True, True),
+               (1536, 3, 2049, True, False), (1536, 4, 4097, False, True), (1528, 6, 1100, False, True),
+               (1536, 7, 1025, True, True), (1272, 8, 1500, True, False), (1536, 9, 3001, False, True)]
+
+
+@pytest.mark.parametrize("D,S,N,separate,with_gain", ROUTE_CASES, ids=[f"D{c[0]}-S{c[1]}-N{c[2]}" for c in ROUTE_CASES])
+def test_narrow_routing_matches_oracle_and_workgroup_kernel(gpu, D, S, N, separate, with_gain):
+    print(f"narrow routing D={D} S={S} N={N}", flush=True)
+    assert route_kernel(S, N, D, 1) == f"attnres_route_rows_c3_s{S}"
+    g = torch.Generator(device=gpu).manual_seed(D + S + N)
+    bf, canary, pad_in, pad_out = torch.bfloat16, 7.0, 64, 32
+    big = torch.full((S + 1, N, D + pad_in), canary, device=gpu, dtype=bf)
+    rows = [big[s] for s in range(S)]
+    if separate:  # not equally spaced
+        rows = [big[s] for s in [S, *range(S - 1)]]
+    for s, r in enumerate(rows):
+        r[:, :D] = (torch.randn((N, D), generator=g, device=gpu) * (0.3 + 0.4 * s)).to(bf)
+    query = (torch.randn(D, generator=g, device=gpu) * 0.05).to(bf)
+    gain = (1 + 0.1 * torch.randn(D, generator=g, device=gpu)).to(bf) if with_gain else None
+
+    def call():
+        out = torch.full((N, D + pad_out), canary, device=gpu, dtype=bf)
+        w, lse = torch.empty((S, N), device=gpu), torch.empty(N, device=gpu)
+        inv, lg = torch.empty((N, S), device=gpu), torch.empty((N, S), device=gpu)
+        _capi.route_fwd(_capi.pointer_array([r.data_ptr() for r in rows]), S, N, D, D + pad_in, _capi.DTYPE_BF16,
+                        query.data_ptr(), None if gain is None else gain.data_ptr(), 1, _capi.DTYPE_BF16, 1e-5,
+                        out.data_ptr(), _capi.DTYPE_BF16, D + pad_out, N * (D + pad_out), w.data_ptr(),
+                        lse.data_ptr(), inv.data_ptr(), lg.data_ptr(), torch.cuda.current_stream(gpu).cuda_stream)
+        torch.cuda.synchronize()
+        assert (out[:, D:] == canary).all(), "output padding written"
+        return out[:, :D], w, lse, inv, lg
+
+    out, w, lse, inv, lg = call()
+    pick = np.unique(np.concatenate([np.arange(0, 64), np.arange(N // 2, N // 2 + 64), np.arange(N - 64, N)]))
+    qw = np64(query) if gain is None else np64(query * gain)  # rounded to bf16, as the kernels fold it
+    ref = O.route(np.stack([np64(r[pick, :D]) for r in rows]), qw, 1e-5)
+    check_bf16(out[pick], ref["out"][0], f"D={D} S={S}")
+    check_weights(w[:, pick], ref["weights"][0], f"D={D} S={S}")
+    np.testing.assert_allclose(np64(lse[pick]), ref["lse"][0], rtol=1e-5, atol=1e-5)
+    np.testing.assert_allclose(np64(inv[pick]), ref["inv_rms"], rtol=1e-5)
+    np.testing.assert_allclose(np64(lg[pick]), ref["logits"][0], rtol=1e-4, atol=1e-4)
+    # every row against the workgroup kernel, with rows of zeros, an infinity, a NaN and the largest
+    # value (whose squares overflow) among them
+    for i, v in enumerate((0.0, math.inf, math.nan, torch.finfo(bf).max)):
+        for r in rows[i % 2:]:
+            r[5 * i, :D if v == 0 else 1] = v
+    mine = call()
+    prev = _capi.set_kernel_policy(_capi.POLICY_WORKGROUP)
+    try:
+        other = call()
+    finally:
+        _capi.set_kernel_policy(prev)
+    for a, b, name in zip(mine, other, ("out", "weights", "lse", "inv_rms", "logits")):
+        a, b = a.double(), b.double()
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf()), name
+        ok = a.isfinite()
+        # bf16 rounding of two fp32 evaluations: one ulp (2^-7 relative) beside the fp32 difference
+        rel, ab = (2.0**-7, 1e-4) if name == "out" else (1e-4, 1e-4)
+        assert ((a - b).abs()[ok] <= rel * b.abs()[ok] + ab).all(), name
