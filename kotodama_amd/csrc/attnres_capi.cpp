@@ -112,7 +112,7 @@ struct DeviceState {
   KernelSlot bwd_stream[2 * 10];  // row-per-wave backward: rows of 6 / 8 KiB x S (1..9)
   KernelSlot bwd_add[kBwdFuncs];   // the same with addend rows (_add)
   KernelSlot bwd_stream_add[2 * 10];
-  KernelSlot bwd_rows[3 * 3 * 10];  // narrow rows' backward: plain / _add / _defer x row KiB (1..3) x S (1..9)
+  KernelSlot bwd_rows[2 * 3 * 10];  // narrow rows' backward: plain / _add x row KiB (1..3) x S (1..9)
   KernelSlot reduce_stage, reduce_cols, reduce_fin;
   KernelSlot merge_bwd[kMergeFuncs];
   KernelSlot merge_bwd_rows[6];  // its row-per-wave form: row KiB (1..6)
@@ -121,7 +121,7 @@ struct DeviceState {
   KernelSlot bwd_dqw_grouped;    // bf16, one chunk per thread, several row groups per workgroup
   KernelSlot bwd_mqg_rows[2 * 2 * 9];  // its row-per-wave form: chunks per lane x query groups x S
   KernelSlot bwd_mqg[2 * 9];     // batched-query backward on the matrix cores: query groups x S
-  KernelSlot bwd_defer[2 * 10];  // row-per-wave backward with deferred block gradients: 6 / 8 KiB rows x S
+  KernelSlot bwd_defer[4 * 10];  // row-per-wave backward with deferred block gradients: row width x S
   KernelSlot gather_seg[4 * ATTNRES_SEG_MAX_BLOCKS];  // segment sums: row width x blocks
 };
 
@@ -447,7 +447,6 @@ int get_bwd_stream(DeviceState& st, int nch, int s, hipFunction_t* f, bool add =
 // KiB even to 1.2 times; at 1024 rows 1.2 times at every width; at 512 even (3
 // KiB rows at S = 9 4% slower) and at 64 rows of 3 KiB 17% slower.
 constexpr int kBwdRowsPart = 11;
-enum BwdRowsVariant { kBwdRowsPlain = 0, kBwdRowsAdd = 1, kBwdRowsDefer = 2 };
 // Row KiB (rounded up) of that kernel for this call, or 0 for another one.
 int bwd_rows_nch(bool bf, bool gbf, int num_sources, int hidden, int64_t num_tokens, int num_cus, bool add) {
   if (!bf || !gbf || hidden > 1536 || num_sources < 1 || num_sources > 9) return 0;
@@ -458,11 +457,10 @@ int bwd_rows_nch(bool bf, bool gbf, int num_sources, int hidden, int64_t num_tok
   const int want = policy == ATTNRES_POLICY_STREAM ? 1 : policy == ATTNRES_POLICY_WORKGROUP ? 0 : tuning().stream;
   return want == 1 || (want < 0 && num_tokens >= 4LL * num_cus) ? nch : 0;
 }
-int get_bwd_rows(DeviceState& st, int nch, int s, BwdRowsVariant var, hipFunction_t* f, int* bpc) {
-  static const char* suffix[] = {"", "_add", "_defer"};
+int get_bwd_rows(DeviceState& st, int nch, int s, bool add, hipFunction_t* f, int* bpc) {
   char name[96];
-  snprintf(name, sizeof(name), "attnres_route_bwd_rows_c%d_s%d%s", nch, s, suffix[var]);
-  return slot_get(st, st.bwd_rows[((int)var * 3 + nch - 1) * 10 + s], kBwdRowsPart, name,
+  snprintf(name, sizeof(name), "attnres_route_bwd_rows_c%d_s%d%s", nch, s, add ? "_add" : "");
+  return slot_get(st, st.bwd_rows[((add ? 3 : 0) + nch - 1) * 10 + s], kBwdRowsPart, name,
                   64 * ATTNRES_ROWS_WAVES, 0, f, bpc);
 }
 // Its grid: two workgroups per CU where they fit (measured in the kernel's comment).
@@ -475,7 +473,7 @@ int bwd_rows_grid(int64_t num_tokens, int num_cus, int bpc, int per_cu = 2) {
 
 // Deferred block gradients (code-object part 10): the row-per-wave backward
 // forming only the partial's gradient (attnres_route_bwd_stream_c<NCH>_s<S>_defer,
-// S >= 2; rows of 1 and 2 KiB: the _defer kernels above) and the sums of the blocks' terms
+// S >= 2) and the sums of the blocks' terms
 // (attnres_route_bwd_gather_seg_c<NCH>_b<NB>).
 constexpr int kDeferPart = 10;
 // The row widths of the deferred path: hidden 3072, 4096, 1024 and 512 (rows of
@@ -1503,7 +1501,7 @@ static int route_bwd_impl(const void* const* sources, int num_sources, int64_t n
   if (rnch > 0) {
     hipFunction_t f = nullptr;
     int bpc = 1;
-    rc = get_bwd_rows(*st, rnch, num_sources, add ? kBwdRowsAdd : kBwdRowsPlain, &f, &bpc);
+    rc = get_bwd_rows(*st, rnch, num_sources, add, &f, &bpc);
     if (rc != ATTNRES_OK) return rc;
     return route_bwd_finish(f, bwd_rows_grid(num_tokens, st->num_cus, bpc), 64 * ATTNRES_ROWS_WAVES, 0, *st,
                             nchunk, sources, num_sources, num_tokens, hidden, src_ld, query, gain, param_dtype, eps,
@@ -1594,20 +1592,6 @@ int attnres_route_bwd_defer(const void* const* sources, int num_sources, int64_t
   DeviceState* st = nullptr;
   int rc = ensure_loaded(&st);
   if (rc != ATTNRES_OK) return rc;
-  void* grads[ATTNRES_MAX_SOURCES] = {};
-  const void* adds[ATTNRES_MAX_SOURCES] = {};
-  grads[num_sources - 1] = grad_partial;
-  adds[num_sources - 1] = grad_partial_addend;
-  if (nch <= 2) {
-    hipFunction_t f = nullptr;
-    int bpc = 1;
-    rc = get_bwd_rows(*st, nch, num_sources, kBwdRowsDefer, &f, &bpc);
-    if (rc != ATTNRES_OK) return rc;
-    return route_bwd_finish(f, bwd_rows_grid(num_tokens, st->num_cus, bpc), 64 * ATTNRES_ROWS_WAVES, 0, *st,
-                            hidden / 8, sources, num_sources, num_tokens, hidden, src_ld, query, gain, param_dtype,
-                            eps, grad_out, grad_out_dtype, grad_out_ld, grad_lse, grads, grad_ld, workspace,
-                            workspace_bytes, grad_query, grad_gain, stream, adds, coef, qfold);
-  }
   if (bwd_stream_lds(nch, num_sources) > (size_t)st->max_lds)
     return fail(ATTNRES_ERR_UNSUPPORTED, "deferred backward: %zu bytes of LDS exceed the device's %d",
                 bwd_stream_lds(nch, num_sources), st->max_lds);
@@ -1615,8 +1599,13 @@ int attnres_route_bwd_defer(const void* const* sources, int num_sources, int64_t
   hipFunction_t f = nullptr;
   rc = get_bwd_defer(*st, nch, num_sources, &f);
   if (rc != ATTNRES_OK) return rc;
+  void* grads[ATTNRES_MAX_SOURCES] = {};
+  const void* adds[ATTNRES_MAX_SOURCES] = {};
+  grads[num_sources - 1] = grad_partial;
+  adds[num_sources - 1] = grad_partial_addend;
   const int64_t need_wg = (num_tokens + kBwdStreamWaves - 1) / kBwdStreamWaves;
-  const int per_cu = tuning().bwd_per_cu > 0 ? tuning().bwd_per_cu : 1;
+  // rows of 1-2 KiB: more waves per CU to keep the memory system busy
+  const int per_cu = tuning().bwd_per_cu > 0 ? tuning().bwd_per_cu : nch <= 2 ? kBwdMaxPerCu : 1;
   const int64_t cap = (int64_t)st->num_cus * per_cu;
   const int grid = (int)(need_wg < cap ? need_wg : cap);
   return route_bwd_finish(f, grid, 64 * kBwdStreamWaves, lds, *st, hidden / 8, sources, num_sources, num_tokens,

@@ -2629,14 +2629,16 @@ __device__ __forceinline__ void rows_query_partial(const float4* dq_lds, float* 
 // rows against a workgroup per row: 1 KiB rows S = 2 26.6 -> 15.0 us, S = 5 41.2
 // -> 23.4, S = 8 54.3 -> 34.2; 1.5 KiB S = 5 48.9 -> 32.4; 2 KiB S = 5 52.7 ->
 // 41.5; 3 KiB S = 5 58.8 -> 57.8, at 32768 rows 252.6 -> 210 (4.2-5.3 TB/s).
-// DEFER at 1 KiB rows, 8192 rows, against route_bwd_stream_body's: S = 2 12.4 ->
-// 11.4 us, S = 5 17.3 -> 15.5.
+// The deferred form of these rows stays with route_bwd_stream_body: here, with
+// the sums in another order, it measured 8-10% faster (1 KiB rows, 8192 rows:
+// S = 2 11.4 against 12.4 us, S = 5 15.5 against 17.3), but moved a training
+// step's gradients by 1.5e-3, no nearer to float64, and runs are continued
+// across builds.
 // Rows are addressed through buffer resources of the row's bytes, so the
 // chunks past the end of a row that is not whole KiB read zeros and their
-// stores are dropped.  ADD and DEFER as in route_bwd_stream_body.
-template <int S, int NCH, bool ADD = false, bool DEFER = false>
+// stores are dropped.  ADD as in route_bwd_stream_body.
+template <int S, int NCH, bool ADD = false>
 __device__ __forceinline__ void route_bwd_rows_body(const attnres_route_bwd_params& P) {
-  static_assert(!DEFER || (ADD && S >= 2), "deferred gradients need a committed source and the addend path");
   constexpr int NV = 3 * S;  // sum(x^2), x.qw, x.G per source
   constexpr int H2 = (NV + 3) / 4;
   constexpr int NP = 4 * H2;
@@ -2666,12 +2668,6 @@ __device__ __forceinline__ void route_bwd_rows_body(const attnres_route_bwd_para
           qw[c][e] = P.param_bf16 ? round_bf16(prod) : prod;
         }
       }
-      if constexpr (DEFER) {
-        if (blockIdx.x == 0 && wave == 0)
-          stg<u32x4>(static_cast<char*>(P.qfold) + (size_t)i * 16,
-                     u32x4{pack_bf16(qw[c][0], qw[c][1]), pack_bf16(qw[c][2], qw[c][3]),
-                           pack_bf16(qw[c][4], qw[c][5]), pack_bf16(qw[c][6], qw[c][7])});
-      }
     }
   }
 
@@ -2699,17 +2695,17 @@ __device__ __forceinline__ void route_bwd_rows_body(const attnres_route_bwd_para
 #pragma unroll
       for (int c = 0; c < NCH; ++c) x[s][c] = ld_row_nt(sr, lane_off + (uint32_t)(c * 1024));
     }
-    // the addend rows (empty resources read zeros): DEFER has the last source's only
-    u32x4 ad[ADD ? (DEFER ? 1 : S) : 1][ADD ? NCH : 1];
+    // the addend rows (empty resources read zeros)
+    u32x4 ad[ADD ? S : 1][ADD ? NCH : 1];
     if constexpr (ADD) {
 #pragma unroll
-      for (int s = DEFER ? S - 1 : 0; s < S; ++s) {
+      for (int s = 0; s < S; ++s) {
         const void* abase = P.dadd[s];
         char* row = const_cast<char*>(
             uniform_ptr(reinterpret_cast<uint64_t>(abase) + (uint64_t)t * ((uint64_t)P.dsrc_ld * 2)));
         const __amdgpu_buffer_rsrc_t ar = row_rsrc(row, abase != nullptr ? row_size : 0u);
 #pragma unroll
-        for (int c = 0; c < NCH; ++c) ad[DEFER ? 0 : s][c] = ld_row_nt(ar, lane_off + (uint32_t)(c * 1024));
+        for (int c = 0; c < NCH; ++c) ad[s][c] = ld_row_nt(ar, lane_off + (uint32_t)(c * 1024));
       }
     }
     const float glse = P.grad_lse != nullptr ? ld_scalar_f32(P.grad_lse + t) : 0.f;
@@ -2761,12 +2757,6 @@ __device__ __forceinline__ void route_bwd_rows_body(const attnres_route_bwd_para
       c1[s] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, c1l), s));
       c2[s] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, c2l), s));
     }
-    if constexpr (DEFER) {
-      // lanes >= S-1 fall outside the resource's range: their stores are dropped
-      char* crow = const_cast<char*>(uniform_ptr(reinterpret_cast<uint64_t>(P.coef) + (uint64_t)t * ((S - 1) * 16)));
-      st_row_nt(row_rsrc(crow, (uint32_t)((S - 1) * 16)), lane_off,
-                u32x4{as_u32(wl), as_u32(c1l), as_u32(c2l), 0u});
-    }
 
     // ---- the gradient rows and the query gradient ----
 #pragma unroll
@@ -2774,17 +2764,6 @@ __device__ __forceinline__ void route_bwd_rows_body(const attnres_route_bwd_para
       // re-expanded from the packed words (opaque), not kept unpacked
 #pragma unroll
       for (int c = 0; c < NCH; ++c) asm volatile("" : "+v"(x[s][c]));
-      if (DEFER && s < S - 1) {
-#pragma unroll
-        for (int c = 0; c < NCH; ++c) {
-#pragma unroll
-          for (int w = 0; w < 4; ++w) {
-            dq[c][2 * w] = __builtin_fmaf(c1[s], bf_lo(x[s][c][w]), dq[c][2 * w]);
-            dq[c][2 * w + 1] = __builtin_fmaf(c1[s], bf_hi(x[s][c][w]), dq[c][2 * w + 1]);
-          }
-        }
-        continue;
-      }
       const __amdgpu_buffer_rsrc_t dr = row_at(P.dsrc[s], P.dsrc_ld, t);
 #pragma unroll
       for (int c = 0; c < NCH; ++c) {
@@ -2798,8 +2777,8 @@ __device__ __forceinline__ void route_bwd_rows_body(const attnres_route_bwd_para
           dq[c][2 * w] = __builtin_fmaf(c1[s], x0, dq[c][2 * w]);
           dq[c][2 * w + 1] = __builtin_fmaf(c1[s], x1, dq[c][2 * w + 1]);
           if constexpr (ADD) {
-            d0 += bf_lo(ad[DEFER ? 0 : s][c][w]);
-            d1 += bf_hi(ad[DEFER ? 0 : s][c][w]);
+            d0 += bf_lo(ad[s][c][w]);
+            d1 += bf_hi(ad[s][c][w]);
           }
           pk[w] = pack_bf16(d0, d1);
         }
@@ -4690,12 +4669,17 @@ BWD_STREAM_ONE_DEFER(8, 6, 0)
 BWD_STREAM_ONE_DEFER(2, 8, 0) BWD_STREAM_ONE_DEFER(3, 8, 0) BWD_STREAM_ONE_DEFER(4, 8, 0)
 BWD_STREAM_ONE_DEFER(5, 8, 0) BWD_STREAM_ONE_DEFER(6, 8, 0) BWD_STREAM_ONE_DEFER(7, 8, 1)
 BWD_STREAM_ONE_DEFER(8, 8, 2) BWD_STREAM_ONE_DEFER(9, 8, 3)
+BWD_STREAM_ONE_DEFER(2, 2, 0) BWD_STREAM_ONE_DEFER(3, 2, 0) BWD_STREAM_ONE_DEFER(4, 2, 0)
+BWD_STREAM_ONE_DEFER(5, 2, 0) BWD_STREAM_ONE_DEFER(6, 2, 0) BWD_STREAM_ONE_DEFER(7, 2, 0)
+BWD_STREAM_ONE_DEFER(8, 2, 0)
+BWD_STREAM_ONE_DEFER(2, 1, 0) BWD_STREAM_ONE_DEFER(3, 1, 0) BWD_STREAM_ONE_DEFER(4, 1, 0)
+BWD_STREAM_ONE_DEFER(5, 1, 0) BWD_STREAM_ONE_DEFER(6, 1, 0) BWD_STREAM_ONE_DEFER(7, 1, 0)
+BWD_STREAM_ONE_DEFER(8, 1, 0)
 #endif
 
 // Row-per-wave backward of narrow rows: attnres_route_bwd_rows_c<NCH>_s<S>, with
-// addend rows (_add) and deferred block gradients (_defer).  Waves per SIMD by
-// the registers a token takes (S + 1 rows of 4 NCH, the query and its gradient
-// 16 NCH, and about 40).
+// addend rows (_add).  Waves per SIMD by the registers a token takes (S + 1 rows
+// of 4 NCH, the query and its gradient 16 NCH, and about 40).
 #define BWD_ROWS_EU(S, NCH, R) \
   (4 * (NCH) * (R) + 16 * (NCH) + 40 <= 128 ? 4 : 4 * (NCH) * (R) + 16 * (NCH) + 40 <= 168 ? 3 : 2)
 #define BWD_ROWS_ONE(S, NCH)                                                                             \
@@ -4709,12 +4693,6 @@ BWD_STREAM_ONE_DEFER(8, 8, 2) BWD_STREAM_ONE_DEFER(9, 8, 3)
       __attribute__((amdgpu_waves_per_eu(BWD_ROWS_EU(S, NCH, 2 * (S) + 1))))                             \
       attnres_route_bwd_rows_c##NCH##_s##S##_add(attnres_route_bwd_params P) {                           \
     route_bwd_rows_body<S, NCH, true>(P);                                                                \
-  }
-#define BWD_ROWS_DEFER(S, NCH)                                                                           \
-  extern "C" __global__ void __launch_bounds__(64 * ATTNRES_ROWS_WAVES)                              \
-      __attribute__((amdgpu_waves_per_eu(BWD_ROWS_EU(S, NCH, (S) + 2))))                                 \
-      attnres_route_bwd_rows_c##NCH##_s##S##_defer(attnres_route_bwd_params P) {                         \
-    route_bwd_rows_body<S, NCH, true, true>(P);                                                          \
   }
 #define MERGE_BWD_ROWS(NCH)                                                                              \
   extern "C" __global__ void __launch_bounds__(64 * ATTNRES_ROWS_WAVES)                              \
@@ -4736,10 +4714,6 @@ BWD_ROWS_ADD(1, 3) BWD_ROWS_ADD(2, 3) BWD_ROWS_ADD(3, 3) BWD_ROWS_ADD(4, 3) BWD_
 ROUTE_ROWS(2, 3) ROUTE_ROWS(3, 3) ROUTE_ROWS(4, 3) ROUTE_ROWS(5, 3)
 ROUTE_ROWS(6, 3) ROUTE_ROWS(7, 3) ROUTE_ROWS(8, 3) ROUTE_ROWS(9, 3)
 MERGE_BWD_ROWS(1) MERGE_BWD_ROWS(2) MERGE_BWD_ROWS(3) MERGE_BWD_ROWS(4) MERGE_BWD_ROWS(5) MERGE_BWD_ROWS(6)
-BWD_ROWS_DEFER(2, 1) BWD_ROWS_DEFER(3, 1) BWD_ROWS_DEFER(4, 1) BWD_ROWS_DEFER(5, 1)
-BWD_ROWS_DEFER(6, 1) BWD_ROWS_DEFER(7, 1) BWD_ROWS_DEFER(8, 1)
-BWD_ROWS_DEFER(2, 2) BWD_ROWS_DEFER(3, 2) BWD_ROWS_DEFER(4, 2) BWD_ROWS_DEFER(5, 2)
-BWD_ROWS_DEFER(6, 2) BWD_ROWS_DEFER(7, 2) BWD_ROWS_DEFER(8, 2)
 #endif
 
 // Segments of deferred sums (the instances in ATTNRES_SEG_INSTANCES), a wave

@@ -19,6 +19,7 @@ read it from those records.  Checked through the C ABI:
 """
 
 import copy
+import hashlib
 
 import numpy as np
 import pytest
@@ -370,3 +371,35 @@ def test_gather_seg_more_terms_than_one_launch(gpu):
     err = np.abs(np64(out) - want)
     bar = bf16_ulp(want) + 0.5 * bf16_ulp(first) + 1e-3 * np.abs(want).max()
     assert (err <= bar).all(), f"{P} terms: worst err {err.max():.3e}"
+
+
+# (S, rows, hidden) -> the digest of the call's outputs.  Rows past one round of the grid, a ragged
+# last round, waves without a row; the values are multiples of powers of two from an integer
+# generator, the same on every host.
+NARROW_DIGESTS = {
+    (2, 8192, 512): "959fb5be9e361d76",
+    (5, 8192, 512): "3d925f0f709fe3e7",
+    (8, 3001, 512): "8dc8ddc729663c5a",
+    (2, 8192, 1024): "121e6bc34f2c3289",
+    (5, 1501, 1024): "c04ff544e00659fb",
+    (8, 4099, 1024): "37a186f9fd18af16",
+}
+
+
+@pytest.mark.parametrize("S,n,d", list(NARROW_DIGESTS), ids=[f"s{c[0]}-n{c[1]}-d{c[2]}" for c in NARROW_DIGESTS])
+def test_narrow_deferred_backward_keeps_its_bits(gpu, S, n, d):
+    # A training run at the proxy's and the 1B model's widths is continued across builds: the order of
+    # this kernel's sums is part of what it returns (another order moves a step's gradients by 1.5e-3).
+    print(f"route_bwd_defer bits S={S} n={n} d={d}", flush=True)
+    g = torch.Generator().manual_seed(S * 10007 + d)
+
+    def ints(lo, hi, scale, *shape):
+        return (torch.randint(lo, hi + 1, shape, generator=g).float() * scale).to(torch.bfloat16).to(gpu)
+
+    srcs = [ints(-127, 127, 2.0 ** (s % 3 - 7), n, d) for s in range(S)]
+    query, gain = ints(-127, 127, 2.0**-10, d), ints(112, 144, 2.0**-7, d)
+    outs = _defer(gpu, srcs, query, gain, ints(-127, 127, 2.0**-6, n, d), ints(-127, 127, 2.0**-6, n, d))
+    h = hashlib.sha256()
+    for t in outs:
+        h.update((t.view(torch.int16) if t.dtype == torch.bfloat16 else t).cpu().numpy().tobytes())
+    assert h.hexdigest()[:16] == NARROW_DIGESTS[S, n, d]
