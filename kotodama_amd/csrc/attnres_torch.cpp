@@ -164,8 +164,8 @@ struct Routed {
 
 // One attnres_route_fwd call; false when the call is not for this path.
 // `squeeze`: one query's rows without the leading query dimension.
-bool route_rows(const Sources& src, const Tensor& query, const Tensor& gain, double eps, at::ScalarType out_dtype,
-                bool want_weights, bool want_lse, bool want_aux, bool squeeze, Routed* r) {
+bool route_rows(const Sources& src, const Tensor& query, const Tensor& gain, double eps,
+                at::ScalarType out_dtype, bool want_weights, bool want_lse, bool want_aux, bool squeeze, Routed* r) {
   if (!src.ok || !dtype_ok(out_dtype)) return false;
   const Fold fold(query, gain, src.d, src.ref);
   if (!fold.ok) return false;
@@ -257,8 +257,12 @@ std::vector<c10::IValue> call_op(const char* name, Args&&... args) {
 std::optional<Tensor> opt(const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; }
 
 // route over a stacked buffer under autograd: the registered op's formula
-// (ops.py: _route_backward, route_bwd) without its Python.
+// (ops.py: _route_backward, route_bwd) without its Python.  Only differentiable
+// outputs (the rows, the lse) pass through the function: compiled autograd
+// takes no function with others.  is_traceable: the backward is made of calls
+// that compiled autograd can trace (under it no call is plain and the ops run).
 struct RouteStacked : public torch::autograd::Function<RouteStacked> {
+  static constexpr bool is_traceable = true;
   static variable_list forward(AutogradContext* ctx, const Tensor& buf, const Tensor& query,
                                const std::optional<Tensor>& gain_opt, const Routed* r, int64_t num, double eps,
                                bool zero_inactive) {
@@ -270,16 +274,9 @@ struct RouteStacked : public torch::autograd::Function<RouteStacked> {
     ctx->saved_data["zero"] = zero_inactive;
     ctx->saved_data["dtype"] = (int64_t)r->out.scalar_type();
     ctx->saved_data["shape"] = r->out.sizes().vec();
-    variable_list out{r->out};
-    variable_list fixed;
-    if (r->lse.defined()) out.push_back(r->lse);
-    for (const Tensor& t : {r->weights, r->inv_rms, r->logits}) {
-      if (!t.defined()) continue;
-      out.push_back(t);
-      fixed.push_back(t);
-    }
-    ctx->mark_non_differentiable(fixed);
     ctx->saved_data["has_lse"] = r->lse.defined();
+    variable_list out{r->out};
+    if (r->lse.defined()) out.push_back(r->lse);
     return out;
   }
 
@@ -325,6 +322,7 @@ struct RouteStacked : public torch::autograd::Function<RouteStacked> {
 
 // The same over a list of separate blocks (ops.py: _route_list_backward, route_list_bwd).
 struct RouteList : public torch::autograd::Function<RouteList> {
+  static constexpr bool is_traceable = true;
   static variable_list forward(AutogradContext* ctx, at::TensorList blocks, const Tensor& query,
                                const std::optional<Tensor>& gain_opt, const Routed* r, double eps) {
     const Tensor gain = gain_opt.value_or(Tensor());
@@ -401,6 +399,7 @@ bool merge_rows(const Tensor& p, const Tensor& query, const Tensor& inter, const
 }
 
 struct Merge : public torch::autograd::Function<Merge> {
+  static constexpr bool is_traceable = true;
   static Tensor forward(AutogradContext* ctx, const Tensor& p, const Tensor& query, const Tensor& inter,
                         const Tensor& lse, const Tensor* out, double eps) {
     ctx->set_materialize_grads(false);
@@ -566,16 +565,15 @@ PyObject* py_route(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Routed r;
   {
     pybind11::gil_scoped_release nogil;
-    if (!route_rows(Sources::stacked(buf, num), query, gain, eps, dt, ww, wl, wa, form == kRows, &r))
+    if (!route_rows(Sources::stacked(buf, num), query, gain, eps, dt, ww, wl, wa, form == kRows,
+                    &r))
       r.out = Tensor();
   }
   if (!r.out.defined()) return none();
   if (rec) {
     const variable_list o = RouteStacked::apply(buf, query, opt(gain), &r, num, eps, a[10] == Py_True);
-    size_t i = 0;
-    r.out = o[i++];
-    for (Tensor* t : {&r.lse, &r.weights, &r.inv_rms, &r.logits})
-      if (t->defined()) *t = o[i++];
+    r.out = o[0];
+    if (r.lse.defined()) r.lse = o[1];
   }
   return pack(r, form);
   END_HANDLE_TH_ERRORS
@@ -604,7 +602,9 @@ PyObject* py_route_list(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Routed r;
   {
     pybind11::gil_scoped_release nogil;
-    if (!route_rows(Sources::list(srcs), query, gain, eps, dt, ww, wl, wa, form == kRows, &r)) r.out = Tensor();
+    if (!route_rows(Sources::list(srcs), query, gain, eps, dt, ww, wl, wa, form == kRows,
+                    &r))
+      r.out = Tensor();
   }
   if (!r.out.defined()) return none();
   if (rec) {

@@ -180,3 +180,48 @@ def test_calls_on_a_side_stream(gpu):
         got = kotodama_amd.route_static(buf, query, Norm(gain), None, 3) + 0
     side.synchronize()
     assert torch.equal(got, want)
+
+
+def _merge_args(gpu):
+    g = torch.Generator(device=gpu).manual_seed(1)
+    return [torch.randn(s, generator=g, device=gpu).to(t).requires_grad_()
+            for s, t in (((2, 9, 264), BF), ((264,), BF), ((2, 9, 264), BF), ((2, 9), F32))]
+
+
+# name -> (tensors, the differentiable output of one recorded call on them)
+RECORDED = {
+    "rows": lambda b, q, g: kotodama_amd.route_static(b, q, Norm(g), None, 2),
+    "all-slots": lambda b, q, g: kotodama_amd.route_static(b, q, Norm(g), None, 3),
+    "weights": lambda b, q, g: ops.route(b, 2, q, g, 1e-5, BF, True, False)[0],
+    "aux": lambda b, q, g: ops.route(b, 2, q, g, 1e-5, BF, False, True)[0],
+    "no-gain": lambda b, q, g: ops.route(b, 2, q, None, 1e-5, BF, False, False)[0] * g,
+    "lse": lambda b, q, g: ops.route_call(b, 2, q, g, 1e-5, BF, want_lse=True)[2],
+    "list": lambda b, q, g: kotodama_amd.block_attn_res_from_list(list(b.unbind(0)), q, Norm(g)),
+    "list-lse": lambda b, q, g: ops.route_list_call(list(b.unbind(0)), q, g, 1e-5, BF, want_lse=True)[2],
+}
+
+
+@pytest.mark.parametrize("name", [*RECORDED, "merge"])
+def test_backward_under_compiled_autograd(gpu, name):
+    # the whole backward is traced (no graph break), once per set of inputs that need gradients
+    def compiler(graph):
+        return torch.compile(graph, backend="aot_eager", fullgraph=True)
+
+    torch._dynamo.reset()
+    for needed in ((0, 1, 2), (0,), (1, 2)):
+        leaves = _merge_args(gpu) if name == "merge" else list(_tensors(gpu))
+        leaves = [t.requires_grad_(i in needed) for i, t in enumerate(leaves)]
+        wanted = [t for t in leaves if t.requires_grad]
+
+        def loss():
+            out = ops.merge_call(*leaves, 1e-5) if name == "merge" else RECORDED[name](*leaves)
+            return out.float().square().sum()
+
+        want = torch.autograd.grad(loss(), wanted)
+        for _ in range(2):
+            for t in wanted:
+                t.grad = None
+            total = loss()
+            with torch._dynamo.compiled_autograd._enable(compiler):
+                total.backward()
+            _same([t.grad for t in wanted], want)
