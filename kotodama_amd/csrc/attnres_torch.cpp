@@ -17,6 +17,7 @@
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/dispatch/Dispatcher.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/record_function.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -156,19 +157,23 @@ struct Sources {
   }
 };
 
+// A profiler's event of a launch that does not pass the dispatcher, under the op's name.
+#define ATTNRES_RECORD(name) RECORD_FUNCTION(name, c10::ArrayRef<const c10::IValue>{})
+
 // ---------------------------------------------------------------- routing --
 
 struct Routed {
   Tensor out, weights, lse, inv_rms, logits;
 };
 
-// One attnres_route_fwd call; false when the call is not for this path.
+// One attnres_route_fwd call, `op` in a profiler; false when the call is not for this path.
 // `squeeze`: one query's rows without the leading query dimension.
-bool route_rows(const Sources& src, const Tensor& query, const Tensor& gain, double eps,
+bool route_rows(const char* op, const Sources& src, const Tensor& query, const Tensor& gain, double eps,
                 at::ScalarType out_dtype, bool want_weights, bool want_lse, bool want_aux, bool squeeze, Routed* r) {
   if (!src.ok || !dtype_ok(out_dtype)) return false;
   const Fold fold(query, gain, src.d, src.ref);
   if (!fold.ok) return false;
+  ATTNRES_RECORD(op);
   const c10::Device dev = src.ref.device();
   const int64_t nq = fold.nq;
   Dims size;
@@ -298,6 +303,7 @@ struct RouteStacked : public torch::autograd::Function<RouteStacked> {
     if (!at::GradMode::is_enabled() && unwatched()) {
       const Sources src = Sources::stacked(buf, num);
       if (src.ok && src.s >= 1 && src.n >= 1) {
+        ATTNRES_RECORD("attnres_hip::route_bwd");
         gb = empty(buf.sizes(), buf.scalar_type(), buf.device());
         const int64_t slot = src.n * src.d * (int64_t)buf.element_size();
         void* grads[ATTNRES_MAX_SOURCES];
@@ -358,6 +364,7 @@ struct RouteList : public torch::autograd::Function<RouteList> {
     if (!at::GradMode::is_enabled() && unwatched()) {
       const Sources src = Sources::list(saved);
       if (src.ok && src.n >= 1) {
+        ATTNRES_RECORD("attnres_hip::route_list_bwd");
         void* ptrs[ATTNRES_MAX_SOURCES];
         for (size_t i = 0; i < s; ++i) {
           grads.push_back(empty(saved[i].sizes(), saved[i].scalar_type(), saved[i].device()));
@@ -391,6 +398,7 @@ bool merge_rows(const Tensor& p, const Tensor& query, const Tensor& inter, const
     return false;
   for (const Tensor* t : {&query, &inter, &lse})
     if (t->get_device() != p.get_device()) return false;
+  ATTNRES_RECORD("attnres_hip::merge");
   *out = empty(inter.sizes(), inter.scalar_type(), inter.device());
   const OnDevice on(p);
   return attnres_merge_fwd(ptr(p), p.numel() / d, (int)d, code(p.scalar_type()), ptr(query), code(query.scalar_type()),
@@ -419,6 +427,7 @@ struct Merge : public torch::autograd::Function<Merge> {
     bool done = false;
     if (!at::GradMode::is_enabled() && unwatched() && n >= 1 && plain(p) && plain(query) && plain(inter) && plain(lse) &&
         dense(go) && go.get_device() == p.get_device() && go.sizes() == inter.sizes()) {
+      ATTNRES_RECORD("attnres_hip::merge_bwd");
       const c10::Device dev = p.device();
       go = go.to(inter.scalar_type()).contiguous();
       gp = empty(p.sizes(), p.scalar_type(), dev);
@@ -565,7 +574,7 @@ PyObject* py_route(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Routed r;
   {
     pybind11::gil_scoped_release nogil;
-    if (!route_rows(Sources::stacked(buf, num), query, gain, eps, dt, ww, wl, wa, form == kRows,
+    if (!route_rows("attnres_hip::route", Sources::stacked(buf, num), query, gain, eps, dt, ww, wl, wa, form == kRows,
                     &r))
       r.out = Tensor();
   }
@@ -602,7 +611,7 @@ PyObject* py_route_list(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Routed r;
   {
     pybind11::gil_scoped_release nogil;
-    if (!route_rows(Sources::list(srcs), query, gain, eps, dt, ww, wl, wa, form == kRows,
+    if (!route_rows("attnres_hip::route_list", Sources::list(srcs), query, gain, eps, dt, ww, wl, wa, form == kRows,
                     &r))
       r.out = Tensor();
   }

@@ -225,3 +225,16 @@ def test_backward_under_compiled_autograd(gpu, name):
             with torch._dynamo.compiled_autograd._enable(compiler):
                 total.backward()
             _same([t.grad for t in wanted], want)
+
+
+def test_recorded_calls_appear_in_a_profile(gpu):
+    buf, query, gain = (t.requires_grad_() for t in _tensors(gpu))
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        RECORDED["rows"](buf, query, gain).float().sum().backward()
+        RECORDED["list"](buf, query, gain).float().sum().backward()
+        ops.merge_call(*_merge_args(gpu), 1e-5).float().sum().backward()
+        with torch.no_grad():
+            ops.route(buf, 3, query, gain, 1e-5, BF, True, False)
+    seen = {e.key: e.count for e in prof.key_averages() if e.key.startswith("attnres_hip::")}
+    names = {f"attnres_hip::{n}": 1 for n in ("route", "route_bwd", "route_list", "route_list_bwd", "merge", "merge_bwd")}
+    assert seen == {**names, "attnres_hip::route": 2}
