@@ -12,8 +12,8 @@ Steps (all outputs under ``kotodama_amd/lib/``):
    the dynamic linker binds that soname to the HIP runtime torch already
    loaded, so streams and device memory are shared with torch.
 5. ``g++`` compiles ``csrc/attnres_torch.cpp`` against torch's headers into
-   ``_attnres_torch.so``, the CPython extension through which the eager torch
-   layer calls that library.
+   ``_attnres_torch`` (with this Python's extension suffix), the CPython
+   extension through which the eager torch layer calls that library.
 
 Run ``python -m kotodama_amd.build`` or call :func:`build`.
 """
@@ -25,6 +25,7 @@ import os
 import subprocess
 import sys
 import tempfile
+from importlib.machinery import EXTENSION_SUFFIXES
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -32,7 +33,7 @@ CSRC = PKG / "csrc"
 LIBDIR = PKG / "lib"
 INCLUDE = PKG.parent / "include"
 LIB_NAME = "libattnres_hip.so"
-NATIVE_NAME = "_attnres_torch.so"
+NATIVE_NAME = "_attnres_torch" + EXTENSION_SUFFIXES[0]  # as _native.py looks it up
 ROCM = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
 ARCH = "gfx950"
 NUM_PARTS = 12
@@ -55,11 +56,12 @@ def _native_cmd(out: Path) -> list[str]:
     """Compile the torch layer's extension to an object file (the link follows the C-ABI library's)."""
     import sysconfig
 
+    import torch
     from torch.utils.cpp_extension import include_paths
 
     incs = [f"-isystem{p}" for p in [*include_paths(), ROCM / "include", sysconfig.get_paths()["include"]]]
     return ["g++", "-c", "-fPIC", "-O2", "-std=c++17", "-Wall", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__",
-            "-DUSE_ROCM", f"-I{INCLUDE}", *incs, str(CSRC / "attnres_torch.cpp"), "-o", str(out)]
+            "-DUSE_ROCM", f'-DATTNRES_TORCH_VERSION="{torch.__version__}"', f"-I{INCLUDE}", *incs, str(CSRC / "attnres_torch.cpp"), "-o", str(out)]
 
 
 def _run(cmd: list[str], cwd: Path | None = None) -> None:

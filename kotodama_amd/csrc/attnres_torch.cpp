@@ -906,4 +906,9 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_attnres_torch", nullptr, -1, kMe
 
 }  // namespace
 
-extern "C" __attribute__((visibility("default"))) PyObject* PyInit__attnres_torch() { return PyModule_Create(&kModule); }
+extern "C" __attribute__((visibility("default"))) PyObject* PyInit__attnres_torch() {
+  PyObject* mod = PyModule_Create(&kModule);
+  // the torch this was compiled for: the loader takes no other (_native.py)
+  if (mod != nullptr && PyModule_AddStringConstant(mod, "torch_version", ATTNRES_TORCH_VERSION) != 0) Py_CLEAR(mod);
+  return mod;
+}
