@@ -11,16 +11,17 @@ Steps (all outputs under ``kotodama_amd/lib/``):
    shared library, linked against ROCm's ``libamdhip64.so.7``.  Loaded after ``import torch``,
    the dynamic linker binds that soname to the HIP runtime torch already
    loaded, so streams and device memory are shared with torch.
-5. ``g++`` compiles ``csrc/attnres_torch.cpp`` against torch's headers into
-   ``_attnres_torch`` (with this Python's extension suffix), the CPython
-   extension through which the eager torch layer calls that library.
+5. Where a ROCm torch is importable, ``g++`` compiles ``csrc/attnres_torch.cpp``
+   against its headers into ``_attnres_torch`` (with this Python's extension
+   suffix), the CPython extension through which the eager torch layer calls
+   that library.  The library needs no torch and is in place before this step
+   can fail; an extension of an earlier build does not stay beside it.
 
 Run ``python -m kotodama_amd.build`` or call :func:`build`.
 """
 
 from __future__ import annotations
 
-import importlib.util
 import os
 import subprocess
 import sys
@@ -52,22 +53,37 @@ HIP_FLAGS = [
 ]
 
 
-def _native_cmd(out: Path) -> list[str]:
+def _rocm_torch():
+    """The torch module the extension can be built against, or None (no torch, or not a ROCm one)."""
+    try:
+        import torch
+    except ImportError:
+        return None
+    return torch if torch.version.hip is not None else None
+
+
+def _native_cmd(torch, out: Path) -> list[str]:
     """Compile the torch layer's extension to an object file (the link follows the C-ABI library's)."""
     import sysconfig
 
-    import torch
     from torch.utils.cpp_extension import include_paths
 
     incs = [f"-isystem{p}" for p in [*include_paths(), ROCM / "include", sysconfig.get_paths()["include"]]]
     return ["g++", "-c", "-fPIC", "-O2", "-std=c++17", "-Wall", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__",
-            "-DUSE_ROCM", f'-DATTNRES_TORCH_VERSION="{torch.__version__}"', f"-I{INCLUDE}", *incs, str(CSRC / "attnres_torch.cpp"), "-o", str(out)]
+            "-DUSE_ROCM", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+            f'-DATTNRES_TORCH_VERSION="{torch.__version__}"', f"-I{INCLUDE}", *incs, str(CSRC / "attnres_torch.cpp"), "-o", str(out)]
 
 
 def _run(cmd: list[str], cwd: Path | None = None) -> None:
     res = subprocess.run(cmd, cwd=cwd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"build step failed ({res.returncode}): {' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
+
+
+def _wait(cmd: list[str], proc: subprocess.Popen) -> None:
+    so, se = proc.communicate()
+    if proc.returncode != 0:
+        raise RuntimeError(f"{Path(cmd[0]).name} failed ({proc.returncode}): {' '.join(cmd)}\n{so}\n{se}")
 
 
 def build(verbose: bool = False, out_dir: Path | None = None, defines: tuple = ()) -> Path:
@@ -84,10 +100,10 @@ def build(verbose: bool = False, out_dir: Path | None = None, defines: tuple = (
         tmpd = Path(tmp)
         procs = []
         native_o = tmpd / "attnres_torch.o"
-        with_torch = importlib.util.find_spec("torch") is not None  # the C-ABI library needs no torch
-        if with_torch:
-            native = _native_cmd(native_o)
-            procs.append((native, subprocess.Popen(native, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)))
+        torch = _rocm_torch()
+        if torch is not None:
+            native = _native_cmd(torch, native_o)
+            native_proc = subprocess.Popen(native, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)
         for part in range(NUM_PARTS):
             out = tmpd / f"attnres_gfx950_part{part}.hsaco"
             cmd = [hipcc, *HIP_FLAGS, *extra, f"-DATTNRES_PART={part}", f"-I{CSRC}", str(CSRC / "attnres_kernels.hip"),
@@ -96,9 +112,7 @@ def build(verbose: bool = False, out_dir: Path | None = None, defines: tuple = (
                 print(" ".join(cmd), flush=True)
             procs.append((cmd, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)))
         for cmd, p in procs:
-            so, se = p.communicate()
-            if p.returncode != 0:
-                raise RuntimeError(f"{Path(cmd[0]).name} failed ({p.returncode}): {' '.join(cmd)}\n{so}\n{se}")
+            _wait(cmd, p)
         blob_o = tmpd / "attnres_blob.o"
         _run(["gcc", "-c", f"-I{tmpd}", str(CSRC / "attnres_blob.S"), "-o", str(blob_o)])
         noalloc_o = tmpd / "attnres_noalloc.o"
@@ -133,9 +147,10 @@ def build(verbose: bool = False, out_dir: Path | None = None, defines: tuple = (
         )
         final = libdir / LIB_NAME
         os.replace(so_tmp, final)  # atomic: a reader never sees a half-written library
-        if with_torch:
-            import torch
-
+        for old in libdir.glob("_attnres_torch*.so"):
+            old.unlink()  # made for the library that was here before
+        if torch is not None:
+            _wait(native, native_proc)
             torch_lib = Path(torch.__file__).parent / "lib"
             native_tmp = tmpd / NATIVE_NAME
             _run(["g++", "-shared", str(native_o), f"-L{libdir}", "-lattnres_hip", f"-L{torch_lib}", "-ltorch_python",

@@ -1,8 +1,11 @@
-"""The native extension's loading, on the CPU: what is there but does not fit
-leaves the ctypes path in place."""
+"""The native extension's loading and building, on the CPU: what is there but
+does not fit leaves the ctypes path in place, and the C-ABI library does not
+depend on it."""
 
 import subprocess
+import sys
 import types
+from pathlib import Path
 
 import pytest
 import torch
@@ -65,3 +68,60 @@ def test_names_agree_and_the_built_extension_loads(monkeypatch):
     assert mod.torch_version == torch.__version__
     assert all(callable(getattr(mod, fn)) for fn in _native.FUNCTIONS)
     assert mod.route(1, 2) is None  # not a call it takes
+
+
+class _Proc:
+    def __init__(self, cmd, fails, **kw):
+        self.returncode = int(fails(cmd))
+        if not self.returncode:
+            Path(cmd[cmd.index("-o") + 1]).write_bytes(b"built")
+
+    def communicate(self):
+        return "", "c10/hip headers are missing"
+
+
+def _fake_build(monkeypatch, out, fails=lambda cmd: False):
+    cmds = []
+
+    def start(cmd, **kw):
+        cmds.append(cmd)
+        return _Proc(cmd, fails, **kw)
+
+    def run(cmd, cwd=None):
+        kbuild._wait(cmd, start(cmd))
+
+    monkeypatch.setattr(kbuild.subprocess, "Popen", start)
+    monkeypatch.setattr(kbuild, "_run", run)
+    kbuild.build(out_dir=out)
+    return cmds
+
+
+def test_library_is_in_place_when_the_extension_does_not_compile(monkeypatch, tmp_path):
+    stale = tmp_path / "_attnres_torch.so"
+    stale.write_bytes(b"an earlier build")
+    with pytest.raises(RuntimeError, match="headers are missing"):
+        _fake_build(monkeypatch, tmp_path, lambda cmd: any("attnres_torch.cpp" in str(c) for c in cmd))
+    assert (tmp_path / kbuild.LIB_NAME).read_bytes() == b"built"
+    assert not stale.exists()
+
+
+@pytest.mark.parametrize("torch_there", ["cpu-only", "none"])
+def test_library_needs_no_rocm_torch(monkeypatch, tmp_path, torch_there):
+    (tmp_path / kbuild.NATIVE_NAME).write_bytes(b"an earlier build")
+    if torch_there == "none":
+        monkeypatch.setitem(sys.modules, "torch", None)  # import torch fails
+    else:
+        monkeypatch.setattr(torch.version, "hip", None)
+    cmds = _fake_build(monkeypatch, tmp_path)
+    assert [p.name for p in tmp_path.iterdir()] == [kbuild.LIB_NAME]
+    assert not any("attnres_torch" in str(c) for cmd in cmds for c in cmd)
+
+
+def test_extension_is_built_for_this_torch_and_python(monkeypatch, tmp_path):
+    if torch.version.hip is None:
+        pytest.skip("not a ROCm torch")
+    cmds = _fake_build(monkeypatch, tmp_path)
+    assert (tmp_path / kbuild.NATIVE_NAME).read_bytes() == b"built"
+    (compile_cmd,) = [c for c in cmds if any("attnres_torch.cpp" in a for a in c)]
+    assert f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}" in compile_cmd
+    assert f'-DATTNRES_TORCH_VERSION="{torch.__version__}"' in compile_cmd
