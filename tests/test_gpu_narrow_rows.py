@@ -146,6 +146,38 @@ def test_row_per_wave_batched_backward_matches_oracle(gpu, D, S, N, Q):
     check_grad(buf.grad.reshape(S, N, D), dx, torch.bfloat16, "dsources")
 
 
+# (hidden, sources, rows, queries, gain) of the grouped query-gradient pass: exactly 64 KiB of sums,
+# two and three row groups that each walk several rows, a second pass over a ragged last query with
+# the per-query reduction
+GROUPED_CASES = [(2048, 4, 2051, 8, False), (1288, 3, 3001, 5, True), (1024, 3, 1030, 9, False),
+                 (1024, 2, 700, 9, True)]
+
+
+@pytest.mark.parametrize("D,S,N,Q,with_gain", GROUPED_CASES,
+                         ids=[f"D{c[0]}-S{c[1]}-N{c[2]}-Q{c[3]}" for c in GROUPED_CASES])
+def test_grouped_query_gradients_match_oracle(gpu, D, S, N, Q, with_gain):
+    print(f"grouped query gradients D={D} S={S} N={N} Q={Q}", flush=True)
+    g = torch.Generator(device="cpu").manual_seed(D + S + N)
+    bf = torch.bfloat16
+    buf = torch.randn(S, 1, N, D, generator=g).to(bf).to(gpu)
+    qs = (torch.randn(Q, D, generator=g) * 0.05).to(bf).to(gpu).requires_grad_()
+    gain = (1 + 0.1 * torch.randn(D, generator=g)).to(bf).to(gpu).requires_grad_() if with_gain else None
+    G = torch.randn(Q, 1, N, D, generator=g).to(bf).to(gpu)
+    buf.requires_grad_()
+    out = ops.route_call(buf, S, qs, gain, 1e-5, bf)[0]
+    out.backward(G)
+    x, dx, dgain = np64(buf).reshape(S, N, D), 0, 0
+    for j in range(Q):
+        b = O.route_backward(x, O.fold_query(np64(qs[j]), np64(gain) if with_gain else None, "bf16"), 1e-5,
+                             np64(G[j]).reshape(N, D))
+        dx = dx + b["dx"]
+        dgain = dgain + b["dqw"] * np64(qs[j])
+        check_grad(qs.grad[j], b["dqw"] * (np64(gain) if with_gain else 1.0), bf, f"dquery[{j}]")
+    check_grad(buf.grad.reshape(S, N, D), dx, bf, "dsources")
+    if with_gain:
+        check_grad(gain.grad, dgain, bf, "dgain")
+
+
 FORWARD_MERGE_CASES = [(8, 1024, None), (504, 1025, None), (520, 3001, torch.float32), (1536, 1030, None)]
 
 
@@ -243,3 +275,75 @@ def test_narrow_routing_matches_oracle_and_workgroup_kernel(gpu, D, S, N, separa
         # bf16 rounding of two fp32 evaluations: one ulp (2^-7 relative) beside the fp32 difference
         rel, ab = (2.0**-7, 1e-4) if name == "out" else (1e-4, 1e-4)
         assert ((a - b).abs()[ok] <= rel * b.abs()[ok] + ab).all(), name
+
+
+def _odd_rows(*bufs):
+    """Rows of zeros, an infinity, a NaN and the largest value (whose squares overflow) into (n, D) rows."""
+    for i, v in enumerate((0.0, math.inf, math.nan, torch.finfo(torch.bfloat16).max)):
+        for r in bufs:
+            r[5 * i, : r.shape[1] if v == 0 else 1] = v
+
+
+def _agree(mine, other, rel, names):
+    """Infinities and NaN in the same places, and every finite value within ``rel`` of the other's."""
+    for a, b, r, name in zip(mine, other, rel, names):
+        a, b = a.double(), b.double()
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf()), name
+        ok = b.isfinite()
+        assert ((a - b).abs()[ok] <= r * b.abs()[ok] + 1e-4).all(), name
+
+
+def _both_policies(call):
+    res = []
+    for policy in (_capi.POLICY_AUTO, _capi.POLICY_WORKGROUP):
+        prev = _capi.set_kernel_policy(policy)
+        try:
+            res.append(call())
+        finally:
+            _capi.set_kernel_policy(prev)
+    return res
+
+
+# one bf16 ulp (2^-7 relative) between the roundings of two fp32 evaluations
+ULP = 2.0**-7
+
+
+@pytest.mark.parametrize("D,S,N", [(520, 5, 1030), (1024, 9, 1100), (1536, 3, 1026)])
+@pytest.mark.parametrize("add", [False, True], ids=["plain", "add"])
+def test_narrow_backward_of_odd_values_as_the_workgroup_kernel(gpu, D, S, N, add):
+    print(f"narrow backward, odd values D={D} S={S} N={N} add={add}", flush=True)
+    assert _bwd_kernel_name(S, N, D, _capi.POLICY_AUTO) == f"attnres_route_bwd_rows_c{(D + 511) // 512}_s{S}"
+    src, q, gain, gout, addend = _case(gpu, S, N, D, torch.bfloat16, 40 + S)
+    _odd_rows(*src[::2])
+    gout[25, 0], gout[30, 0] = math.inf, math.nan
+
+    def call():
+        grads = torch.zeros_like(src)
+        dq, dg = _call(gpu, src, q, gain, gout, grads, list(addend) if add else None)
+        return grads, dq, dg
+
+    mine, other = _both_policies(call)
+    assert mine[0].isnan().any() and mine[0].isfinite().any()
+    _agree(mine, other, [ULP] * 3, ["dsources", "dquery", "dgain"])
+
+
+@pytest.mark.parametrize("D,N", [(520, 1030), (1536, 1026)])
+def test_narrow_merge_of_odd_values_as_the_workgroup_kernel(gpu, D, N):
+    print(f"narrow merge, odd values D={D} N={N}", flush=True)
+    bf = torch.bfloat16
+    assert merge_kernel(N, D, bf) == f"attnres_merge_rows_c{(D + 511) // 512}"
+    g = torch.Generator(device=gpu).manual_seed(D)
+    p, inter, G = (torch.randn((N, D), generator=g, device=gpu).to(bf) for _ in range(3))
+    q, lse = (torch.randn(D, generator=g, device=gpu) * 0.1).to(bf), torch.randn(N, generator=g, device=gpu)
+    _odd_rows(p)
+    inter[25, 0], inter[30, 0], lse[35], lse[40], lse[45] = math.inf, math.nan, math.inf, -math.inf, math.nan
+    G[50, 0], G[55, 0] = math.inf, math.nan
+
+    def call():
+        leaves = [t.clone().requires_grad_() for t in (p, q, inter, lse)]
+        out = ops.merge_call(*leaves, 1e-5)
+        return [out.detach(), *torch.autograd.grad(out, leaves, G)]
+
+    mine, other = _both_policies(call)
+    assert mine[0].isnan().any() and mine[0].isfinite().any()
+    _agree(mine, other, [ULP] * 4 + [1e-4], ["out", "dpartial", "dquery", "dinter", "dlse"])

@@ -10,6 +10,8 @@ import kotodama_amd
 from kotodama_amd import ops
 from kotodama_amd._native import native
 
+from ._tiny_model import TinyModel
+
 pytestmark = pytest.mark.gpu
 BF, F32 = torch.bfloat16, torch.float32
 OP = torch.ops.attnres_hip
@@ -70,21 +72,37 @@ def test_forward_forms_equal_the_ops(gpu, form, with_gain):
 
 @pytest.mark.parametrize("form", FORMS, ids=[",".join(f"{k}={v}" for k, v in f.items()) or "plain" for f in FORMS])
 @pytest.mark.parametrize("stacked", [True, False], ids=["stacked", "list"])
-def test_gradients_equal_the_ops(gpu, form, stacked):
+@pytest.mark.parametrize("used", ["rows", "lse", "both", "rows of both"])
+def test_gradients_equal_the_ops(gpu, form, stacked, used):
+    want_lse = used != "rows"
+    weights = [False, True] if stacked and want_lse else [False]  # a recorded list call with weights is the op's
     res = []
-    for call in ((lambda *a: ops.route(*a)) if stacked else (lambda *a: ops.route_list(*a)),
-                 OP.route if stacked else OP.route_list):
+    for direct in [*weights, None]:  # native, and last the op
         buf, query, gain = _tensors(gpu, **form)
         leaves = [t.requires_grad_() for t in ([buf] if stacked else [b.clone() for b in buf])]
         query.requires_grad_(), gain.requires_grad_()
         # one inactive slot where the buffer has more than one
         n = max(1, buf.shape[0] - 1)
         args = (leaves[0], n) if stacked else (leaves[:n],)
-        out, _, lse, _, _ = call(*args, query, gain, 1e-5, buf.dtype, True, False)
+        if direct is None:
+            call = OP.route if stacked else OP.route_list
+            out, _, lse, _, _ = call(*args, query, gain, 1e-5, buf.dtype, want_lse, False)
+        else:
+            call = native.route if stacked else native.route_list
+            got = call(*args, query, gain, 1e-5, buf.dtype, direct, want_lse, False, ops._TUPLE, True)
+            assert got is not None, "the native path left the call alone"
+            out, w, lse, _, _ = got
+            assert ("RouteStacked" if stacked else "RouteList") in out.grad_fn.name()
+            assert w is None or not w.requires_grad
         g = torch.Generator(device=gpu).manual_seed(5)
-        loss = (out.float() * torch.randn(out.shape, generator=g, device=gpu)).sum() + lse.sum()
+        loss = 0
+        if used != "lse":
+            loss = (out.float() * torch.randn(out.shape, generator=g, device=gpu)).sum()
+        if used in ("lse", "both"):
+            loss = loss + lse.sum()
         res.append(torch.autograd.grad(loss, [*leaves[:n], query, gain]))
-    _same(*res)
+    for got in res[:-1]:
+        _same(got, res[-1])
 
 
 @pytest.mark.parametrize("dtypes", [(BF, BF, BF), (F32, F32, F32), (BF, F32, BF), (F32, BF, F32)])
@@ -236,5 +254,44 @@ def test_recorded_calls_appear_in_a_profile(gpu):
         with torch.no_grad():
             ops.route(buf, 3, query, gain, 1e-5, BF, True, False)
     seen = {e.key: e.count for e in prof.key_averages() if e.key.startswith("attnres_hip::")}
-    names = {f"attnres_hip::{n}": 1 for n in ("route", "route_bwd", "route_list", "route_list_bwd", "merge", "merge_bwd")}
+    names = {f"attnres_hip::{n}{d}": 1 for n in ("route", "route_list", "merge") for d in ("", "_bwd")}
     assert seen == {**names, "attnres_hip::route": 2}
+
+
+class _Recorder:
+    """The native functions, counting the calls taken; with ``off`` none is."""
+
+    def __init__(self, off):
+        self.off, self.taken = off, {}
+
+    def __getattr__(self, name):
+        def call(*args):
+            res = None if self.off else getattr(native, name)(*args)
+            if res is not None:
+                self.taken[name] = self.taken.get(name, 0) + 1
+            return res
+
+        return call
+
+
+# (hidden, dtype, the training points' native functions that the loop must reach)
+LOOPS = [(512, BF, {"step", "bwd_rows", "bwd_defer", "gather_seg"}), (1024, BF, {"step", "bwd_defer", "gather_seg"}),
+         (264, BF, {"step", "bwd_rows"}), (512, F32, {"step", "bwd_rows"})]
+
+
+@pytest.mark.parametrize("d,dtype,reached", LOOPS, ids=[f"d{c[0]}-{str(c[1])[6:]}" for c in LOOPS])
+def test_training_loop_equals_the_python_launches(gpu, monkeypatch, d, dtype, reached):
+    model = TinyModel(d=d, num_layers=6, boundaries=(0, 2, 4), elementwise=True).to(gpu).to(dtype)
+    g = torch.Generator(device=gpu).manual_seed(d)
+    embed = torch.randn((2, 33, d), generator=g, device=gpu).to(dtype).requires_grad_()
+    grad = torch.randn((2, 33, d), generator=g, device=gpu).to(dtype)
+    params = [p for p in model.parameters() if p.requires_grad]
+    res = []
+    for off in (False, True):
+        rec = _Recorder(off)
+        monkeypatch.setattr(ops, "native", rec)
+        out = kotodama_amd.forward_attn_res(model, embed)
+        res.append([out.detach(), *torch.autograd.grad(out, [embed, *params], grad, allow_unused=True)])
+        assert off or reached <= set(rec.taken), rec.taken
+        assert not off or not rec.taken
+    _same(*res)

@@ -128,8 +128,23 @@ def test_route_bwd_row_per_wave_row_strides(gpu, S, n):
         _capi.set_kernel_policy(prev)
 
 
-def _route_bwd_strided(gpu, sdt, S, n, d):
-    print(f"route_bwd strided {sdt} S={S} n={n} d={d}", flush=True)
+@pytest.mark.parametrize("S,n,d,add", [(2, 1029, 512, False), (2, 1029, 512, True), (5, 777, 1000, False),
+                                       (9, 777, 1000, True), (9, 1030, 1536, False), (6, 1100, 1032, True)])
+def test_route_bwd_narrow_rows_row_strides(gpu, S, n, d, add):
+    # the narrow rows' row-per-wave backward: row resources end at the row, not at its stride
+    kn = ctypes.create_string_buffer(128)
+    prev = _capi.set_kernel_policy(_capi.POLICY_STREAM)
+    try:
+        _capi.check("attnres_route_bwd_kernel_name", _capi.lib().attnres_route_bwd_kernel_name(
+            S, n, d, _capi.DTYPE_BF16, _capi.DTYPE_BF16, kn, 128))
+        assert kn.value.decode() == f"attnres_route_bwd_rows_c{(d + 511) // 512}_s{S}"
+        _route_bwd_strided(gpu, torch.bfloat16, S, n, d, add)
+    finally:
+        _capi.set_kernel_policy(prev)
+
+
+def _route_bwd_strided(gpu, sdt, S, n, d, add=False):
+    print(f"route_bwd strided {sdt} S={S} n={n} d={d} add={add}", flush=True)
     src_ld, gout_ld, grad_ld = d + 64, d + 128, d + 32
     g = torch.Generator(device=gpu).manual_seed(S * 7 + (sdt == torch.float32))
     big = torch.full((S, n, src_ld), CANARY, device=gpu, dtype=sdt)
@@ -143,13 +158,20 @@ def _route_bwd_strided(gpu, sdt, S, n, d):
     dbig = torch.full((S, n, grad_ld), CANARY, device=gpu, dtype=sdt)
     ws = torch.empty(_capi.route_bwd_workspace_size(n, d) // 4, device=gpu)
     dq = torch.empty(d, device=gpu, dtype=qdt)
-    _capi.route_bwd(
+    if add:  # the gradient rows of every other source are added to in place
+        dbig[::2, :, :d] = (torch.randn((len(dbig[::2]), n, d), generator=g, device=gpu) * 0.01).to(sdt)
+    addend = np64(dbig[:, :, :d])
+    addend[1::2] = 0
+    adds = (_capi.pointer_array([dbig[s].data_ptr() if s % 2 == 0 else None for s in range(S)]),) if add else ()
+    (_capi.route_bwd_add if add else _capi.route_bwd)(
         _capi.pointer_array([big[s].data_ptr() for s in range(S)]), S, n, d, src_ld, code(sdt), q.data_ptr(), None,
         code(qdt), 1e-5, gbuf.data_ptr(), code(sdt), gout_ld, glse.data_ptr(),
-        _capi.pointer_array([dbig[s].data_ptr() for s in range(S)]), grad_ld, ws.data_ptr(), ws.numel() * 4,
+        _capi.pointer_array([dbig[s].data_ptr() for s in range(S)]), *adds, grad_ld, ws.data_ptr(), ws.numel() * 4,
         dq.data_ptr(), None, torch.cuda.current_stream(gpu).cuda_stream)
     torch.cuda.synchronize()
     ref = O.route_backward(np64(big[:, :, :d]), np64(q), 1e-5, np64(gbuf[:, :d]), np64(glse))
+    if add:
+        ref["dx"] = ref["dx"] + addend
     got = np64(dbig[:, :, :d])
     scale = np.abs(ref["dx"]).max()
     if sdt == torch.float32:
@@ -162,6 +184,52 @@ def _route_bwd_strided(gpu, sdt, S, n, d):
     tq = 1e-4 * np.abs(dqr) + 1e-5 * np.abs(dqr).max() if qdt == torch.float32 else \
         bf16_ulp(dqr) + 1e-3 * np.abs(dqr).max()
     assert (np.abs(np64(dq) - dqr) <= tq).all(), "query gradient"
+
+
+# (S, rows, hidden, queries, kernel): the row-per-wave form with one and two chunks per lane, the
+# row-per-workgroup one; query-gradient passes of four, two and one row groups per workgroup
+QUERY_CASES = [(3, 1029, 504, 5, "mqg_rows_v1_s3_q2"), (8, 777, 1024, 8, "mqg_rows_v2_s8_q2"),
+               (2, 600, 2048, 8, "mqg_s2_q2"), (4, 300, 3072, 3, "mqg_s4_q1")]
+
+
+@pytest.mark.parametrize("S,n,d,Q,kernel", QUERY_CASES, ids=[f"s{c[0]}-n{c[1]}-d{c[2]}-q{c[3]}" for c in QUERY_CASES])
+def test_route_bwd_queries_row_strides(gpu, S, n, d, Q, kernel):
+    print(f"route_bwd_queries strided S={S} n={n} d={d} Q={Q}", flush=True)
+    bf, BF = torch.bfloat16, _capi.DTYPE_BF16
+    kn = ctypes.create_string_buffer(128)
+    _capi.check("attnres_route_bwd_queries_kernel_name",
+                _capi.lib().attnres_route_bwd_queries_kernel_name(S, d, BF, BF, BF, Q, kn, 128))
+    assert kn.value.decode() == f"attnres_route_bwd_{kernel}"
+    src_ld, gout_ld, grad_ld, qstride = d + 64, d + 128, d + 32, n * (d + 128) + 64
+    g = torch.Generator(device=gpu).manual_seed(S * 17 + n)
+    big = torch.full((S, n, src_ld), CANARY, device=gpu, dtype=bf)
+    for s in range(S):
+        big[s, :, :d] = (torch.randn((n, d), generator=g, device=gpu) * (0.5 + 0.3 * s)).to(bf)
+    qs = (torch.randn((Q, d), generator=g, device=gpu) * 0.05).to(bf)
+    gbuf = torch.full((Q * qstride,), CANARY, device=gpu, dtype=bf)
+    G = [gbuf[q * qstride: q * qstride + n * gout_ld].view(n, gout_ld) for q in range(Q)]
+    for v in G:
+        v[:, :d] = torch.randn((n, d), generator=g, device=gpu).to(bf)
+    glse = torch.randn((Q, n), generator=g, device=gpu) * 0.1
+    dbig = torch.full((S, n, grad_ld), CANARY, device=gpu, dtype=bf)
+    ws = torch.empty(_capi.route_bwd_queries_workspace_size(n, d, S, Q) // 4 + 1, device=gpu)
+    dq = torch.empty((Q, d), device=gpu, dtype=bf)
+    rc = _capi.route_bwd_queries(
+        _capi.pointer_array([big[s].data_ptr() for s in range(S)]), S, n, d, src_ld, BF, qs.data_ptr(), None, Q, BF,
+        1e-5, gbuf.data_ptr(), BF, gout_ld, qstride, glse.data_ptr(),
+        _capi.pointer_array([dbig[s].data_ptr() for s in range(S)]), grad_ld, ws.data_ptr(), ws.numel() * 4,
+        dq.data_ptr(), None, torch.cuda.current_stream(gpu).cuda_stream)
+    assert rc == _capi.OK
+    torch.cuda.synchronize()
+    dx = 0
+    for q in range(Q):
+        ref = O.route_backward(np64(big[:, :, :d]), np64(qs[q]), 1e-5, np64(G[q][:, :d]), np64(glse[q]))
+        dx = dx + ref["dx"]
+        want = ref["dqw"]
+        assert (np.abs(np64(dq[q]) - want) <= bf16_ulp(want) + 1e-3 * np.abs(want).max()).all(), f"query gradient {q}"
+    err = np.abs(np64(dbig[:, :, :d]) - dx)
+    assert (err <= bf16_ulp(dx) + 1e-3 * np.abs(dx).max()).all(), f"dx worst err {err.max():.3e}"
+    assert torch.all(dbig[:, :, d:] == CANARY), "gradient row padding written"
 
 
 @pytest.mark.parametrize("S,n,d", [(3, 777, 3072), (9, 515, 4096)])
