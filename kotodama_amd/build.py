@@ -71,7 +71,8 @@ def _native_cmd(torch, out: Path) -> list[str]:
     incs = [f"-isystem{p}" for p in [*include_paths(), ROCM / "include", sysconfig.get_paths()["include"]]]
     return ["g++", "-c", "-fPIC", "-O2", "-std=c++17", "-Wall", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__",
             "-DUSE_ROCM", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
-            f'-DATTNRES_TORCH_VERSION="{torch.__version__}"', f"-I{INCLUDE}", *incs, str(CSRC / "attnres_torch.cpp"), "-o", str(out)]
+            f'-DATTNRES_TORCH_VERSION="{torch.__version__}"', f"-I{INCLUDE}", f"-I{CSRC}", *incs,
+            str(CSRC / "attnres_torch.cpp"), "-o", str(out)]
 
 
 def _run(cmd: list[str], cwd: Path | None = None) -> None:

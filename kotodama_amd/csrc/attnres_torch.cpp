@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "attnres.h"
+#include "attnres_params.h"
 
 namespace {
 
@@ -217,7 +218,8 @@ bool route_rows_bwd(const Sources& src, void* const* grads, const Tensor& query,
   if (!fold.ok || !dense(g_out) || !dtype_ok(g_out.scalar_type()) || g_out.get_device() != src.ref.get_device() ||
       g_out.numel() != fold.nq * src.n * src.d)
     return false;
-  if (g_lse.defined() && (!dense(g_lse) || g_lse.get_device() != src.ref.get_device() || g_lse.numel() != fold.nq * src.n))
+  if (g_lse.defined() &&
+      (!dense(g_lse) || g_lse.get_device() != src.ref.get_device() || g_lse.numel() != fold.nq * src.n))
     return false;
   g_out = g_out.contiguous();
   if (g_lse.defined()) g_lse = g_lse.to(at::kFloat).contiguous();
@@ -393,8 +395,8 @@ struct RouteList : public torch::autograd::Function<RouteList> {
 bool merge_rows(const Tensor& p, const Tensor& query, const Tensor& inter, const Tensor& lse, double eps, Tensor* out) {
   if (!plain(p) || !plain(inter) || !plain(query) || !plain(lse) || p.dim() < 1) return false;
   const int64_t d = p.size(-1);
-  if (d < 1 || inter.sizes() != p.sizes() || query.dim() != 1 || query.size(0) != d || lse.scalar_type() != at::kFloat ||
-      lse.sizes() != p.sizes().slice(0, p.dim() - 1))
+  if (d < 1 || inter.sizes() != p.sizes() || query.dim() != 1 || query.size(0) != d ||
+      lse.scalar_type() != at::kFloat || lse.sizes() != p.sizes().slice(0, p.dim() - 1))
     return false;
   for (const Tensor* t : {&query, &inter, &lse})
     if (t->get_device() != p.get_device()) return false;
@@ -425,8 +427,8 @@ struct Merge : public torch::autograd::Function<Merge> {
     const int64_t d = p.size(-1), n = p.numel() / d;
     Tensor gp, gq, gi, gl, go = g[0];
     bool done = false;
-    if (!at::GradMode::is_enabled() && unwatched() && n >= 1 && plain(p) && plain(query) && plain(inter) && plain(lse) &&
-        dense(go) && go.get_device() == p.get_device() && go.sizes() == inter.sizes()) {
+    if (!at::GradMode::is_enabled() && unwatched() && n >= 1 && plain(p) && plain(query) && plain(inter) &&
+        plain(lse) && dense(go) && go.get_device() == p.get_device() && go.sizes() == inter.sizes()) {
       ATTNRES_RECORD("attnres_hip::merge_bwd");
       const c10::Device dev = p.device();
       go = go.to(inter.scalar_type()).contiguous();
@@ -565,8 +567,8 @@ PyObject* py_route(PyObject*, PyObject* const* a, Py_ssize_t n) {
   double eps = 0;
   at::ScalarType dt;
   if (n != 11 || !take(a[0], false, &buf) || !take(a[1], &num) || !take(a[2], false, &query) ||
-      !take(a[3], true, &gain) || !take(a[4], &eps) || !take_dtype(a[5], buf, query, gain, &dt) || !take(a[6], &ww) || !take(a[7], &wl) || !take(a[8], &wa) ||
-      !take(a[9], &form) || !unwatched())
+      !take(a[3], true, &gain) || !take(a[4], &eps) || !take_dtype(a[5], buf, query, gain, &dt) || !take(a[6], &ww) ||
+      !take(a[7], &wl) || !take(a[8], &wa) || !take(a[9], &form) || !unwatched())
     return none();
   const bool rec = recorded({&buf, &query, &gain});
   if (rec && (a[10] == Py_None || num < 1 || !no_tangent(buf) || !no_tangent(query) || !no_tangent(gain)))
@@ -660,8 +662,8 @@ PyObject* py_block_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t s = nc + (commit ? 1 : 0) + 1;
   const Sources src = Sources::stacked(arena, std::min<int64_t>(s, arena.dim() > 0 ? arena.size(0) : 0));
   if (!src.ok || s < 1 || s > arena.size(0) || query.dim() != 1) return none();
-  if (delta.defined() && (!plain(delta) || delta.scalar_type() != src.dtype || delta.get_device() != arena.get_device() ||
-                          delta.sizes() != arena.sizes().slice(1)))
+  if (delta.defined() && (!plain(delta) || delta.scalar_type() != src.dtype ||
+                          delta.get_device() != arena.get_device() || delta.sizes() != arena.sizes().slice(1)))
     return none();
   const Fold fold(query, gain, src.d, arena);
   if (!fold.ok) return none();
@@ -826,7 +828,7 @@ PyObject* py_gather_seg(PyObject*, PyObject* const* a, Py_ssize_t n) {
       !take(a[3], false, &x) || !take(a[4], true, &addend) || !unwatched())
     return none();
   const Py_ssize_t nt = PyList_GET_SIZE(a[0]), nb = PyList_GET_SIZE(a[1]);
-  constexpr Py_ssize_t kMaxBlocks = 8, kMaxTerms = 48;  // one launch (ATTNRES_SEG_MAX_*)
+  constexpr Py_ssize_t kMaxBlocks = ATTNRES_SEG_MAX_BLOCKS, kMaxTerms = ATTNRES_SEG_MAX_TERMS;  // one launch
   if (nb < 1 || nb > kMaxBlocks || PyList_GET_SIZE(a[2]) != nb || nt < 1 || nt > kMaxTerms || !plain(x) || x.dim() < 1)
     return none();
   const int64_t d = x.size(-1), rows = d > 0 ? x.numel() / d : 0;
@@ -902,7 +904,8 @@ PyMethodDef kMethods[] = {
     {"block_step", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_block_step)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
-PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_attnres_torch", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_attnres_torch", nullptr, -1, kMethods,
+                       nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
 
