@@ -1057,7 +1057,8 @@ int reduce_launch(const ReduceFns& fn, void* workspace, int nparts, int hidden, 
   const bool fits = (int64_t)(nparts + 1024) * width * 4 < (int64_t)1 << 32;
   if (!tuning().reduce_two_stage && fits) {
     // without a gain gradient the queries are independent: one per workgroup
-    if (num_queries > 1 && grad_gain == nullptr) return launch(fn.cols, (hidden + 31) / 32, 1024, R, stream, num_queries);
+    if (num_queries > 1 && grad_gain == nullptr)
+      return launch(fn.cols, (hidden + 31) / 32, 1024, R, stream, num_queries);
     if (num_queries <= 4) return launch(fn.cols, (hidden + 31) / 32, 1024, R, stream);
   }
   if (nparts > 64) {

@@ -547,7 +547,8 @@ __device__ __forceinline__ void route_body(const attnres_route_params& P) {
     if (S > 0 && P.mode != ATTNRES_MODE_PLAIN) {
       const char* drow = reinterpret_cast<const char*>(P.delta) + t * P.delta_ld * C::BYTES;
 #pragma unroll
-      for (int k = 0; k < V; ++k) dvr[k] = ok[k] ? ldg_hint<NT, u32x4>(drow + (int64_t)chunk[k] * 16) : u32x4{0, 0, 0, 0};
+      for (int k = 0; k < V; ++k)
+        dvr[k] = ok[k] ? ldg_hint<NT, u32x4>(drow + (int64_t)chunk[k] * 16) : u32x4{0, 0, 0, 0};
     }
   };
   // Source rows small enough to stay in the L2s (P.src_cached) are read without
@@ -768,17 +769,17 @@ __device__ __forceinline__ void route_body(const attnres_route_params& P) {
 
 // ---------------------------------- row-per-wave routing of narrow rows --
 //
-// One query over bf16 rows of any width up to NCH KiB (3, the only one launched),
-// bf16 parameters and output: one wave per token row, every source row requested
-// at once through buffer resources of the row's bytes (chunks past the row end
-// read zeros, their stores are dropped), the 2S sums reduced by the transposing
-// tree through the wave's own LDS row, the softmax with lane s for source s, no
-// barrier.  Bound by memory: the streaming kernel's chain of one source row after
-// another in a single workgroup per CU, and the workgroup kernel's barriers, left
-// rows of this size waiting (hidden 1536, 5 sources, 32768 rows: 122 -> 98 us,
-// 6.2 TB/s).
-template <int S, int NCH>
+// One query over bf16 rows of any width up to 3 KiB, bf16 parameters and output:
+// one wave per token row, every source row requested at once through buffer
+// resources of the row's bytes (chunks past the row end read zeros, their stores
+// are dropped), the 2S sums reduced by the transposing tree through the wave's
+// own LDS row, the softmax with lane s for source s, no barrier.  Bound by
+// memory: the streaming kernel's chain of one source row after another in a
+// single workgroup per CU, and the workgroup kernel's barriers, left rows of this
+// size waiting (hidden 1536, 5 sources, 32768 rows: 122 -> 98 us, 6.2 TB/s).
+template <int S>
 __device__ __forceinline__ void route_rows_body(const attnres_route_params& P) {
+  constexpr int NCH = 3;  // the row's KiB, rounded up
   constexpr int NV = 2 * S;
   constexpr int H2 = (NV + 3) / 4;
   constexpr int NP = 4 * H2;
@@ -3361,14 +3362,16 @@ __device__ __forceinline__ void route_bwd_mqg_body(const attnres_route_bwd_mq_pa
       char* row = reinterpret_cast<char*>(const_cast<void*>(P.src[s])) + t * row_bytes_ld;
       const __amdgpu_buffer_rsrc_t rs = row_rsrc(row, row_bytes);
 #pragma unroll
-      for (int k = 0; k < V; ++k) x[s][k] = NT ? ld_row_nt(rs, (uint32_t)chunk[k] * 16) : ld_row(rs, (uint32_t)chunk[k] * 16);
+      for (int k = 0; k < V; ++k)
+        x[s][k] = NT ? ld_row_nt(rs, (uint32_t)chunk[k] * 16) : ld_row(rs, (uint32_t)chunk[k] * 16);
     }
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       char* grow = reinterpret_cast<char*>(const_cast<void*>(P.grad_out)) + (q * P.gout_qstride + t * P.gout_ld) * 2;
       const __amdgpu_buffer_rsrc_t rg = row_rsrc(grow, q < nq ? row_bytes : 0u);
 #pragma unroll
-      for (int k = 0; k < V; ++k) gq[q][k] = NT ? ld_row_nt(rg, (uint32_t)chunk[k] * 16) : ld_row(rg, (uint32_t)chunk[k] * 16);
+      for (int k = 0; k < V; ++k)
+        gq[q][k] = NT ? ld_row_nt(rg, (uint32_t)chunk[k] * 16) : ld_row(rg, (uint32_t)chunk[k] * 16);
     }
   };
   const int64_t tok0 = ROWS ? (int64_t)blockIdx.x * RW + wave : (int64_t)blockIdx.x;
@@ -4030,7 +4033,8 @@ __device__ __forceinline__ void merge_bwd_rows_body(const attnres_merge_bwd_para
   const uint32_t row_size = (uint32_t)P.d * 2;
   const uint32_t lane_off = (uint32_t)lane * 16;
   auto row_at = [&](const void* base, uint32_t t) {
-    return row_rsrc(const_cast<char*>(uniform_ptr(reinterpret_cast<uint64_t>(base) + (uint64_t)t * row_size)), row_size);
+    return row_rsrc(const_cast<char*>(uniform_ptr(reinterpret_cast<uint64_t>(base) + (uint64_t)t * row_size)),
+                    row_size);
   };
   auto lane63 = [](float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
@@ -4700,10 +4704,10 @@ BWD_STREAM_ONE_DEFER(8, 1, 0)
       attnres_merge_bwd_rows_c##NCH(attnres_merge_bwd_params P) {                                        \
     merge_bwd_rows_body<NCH>(P);                                                                         \
   }
-#define ROUTE_ROWS(S, NCH)                                                                               \
+#define ROUTE_ROWS(S)                                                                                    \
   extern "C" __global__ void __launch_bounds__(64 * ATTNRES_ROWS_WAVES)                                  \
-      attnres_route_rows_c##NCH##_s##S(attnres_route_params P) {                                         \
-    route_rows_body<S, NCH>(P);                                                                          \
+      attnres_route_rows_c3_s##S(attnres_route_params P) {                                               \
+    route_rows_body<S>(P);                                                                               \
   }
 #define BWD_ROWS_S(S) \
   BWD_ROWS_ONE(S, 1) BWD_ROWS_ONE(S, 2) BWD_ROWS_ONE(S, 3) BWD_ROWS_ADD(S, 1) BWD_ROWS_ADD(S, 2)
@@ -4711,8 +4715,7 @@ BWD_STREAM_ONE_DEFER(8, 1, 0)
 BWD_ROWS_S(1) BWD_ROWS_S(2) BWD_ROWS_S(3) BWD_ROWS_S(4) BWD_ROWS_S(5)
 BWD_ROWS_S(6) BWD_ROWS_S(7) BWD_ROWS_S(8) BWD_ROWS_S(9)
 BWD_ROWS_ADD(1, 3) BWD_ROWS_ADD(2, 3) BWD_ROWS_ADD(3, 3) BWD_ROWS_ADD(4, 3) BWD_ROWS_ADD(5, 3) BWD_ROWS_ADD(6, 3)
-ROUTE_ROWS(2, 3) ROUTE_ROWS(3, 3) ROUTE_ROWS(4, 3) ROUTE_ROWS(5, 3)
-ROUTE_ROWS(6, 3) ROUTE_ROWS(7, 3) ROUTE_ROWS(8, 3) ROUTE_ROWS(9, 3)
+ROUTE_ROWS(2) ROUTE_ROWS(3) ROUTE_ROWS(4) ROUTE_ROWS(5) ROUTE_ROWS(6) ROUTE_ROWS(7) ROUTE_ROWS(8) ROUTE_ROWS(9)
 MERGE_BWD_ROWS(1) MERGE_BWD_ROWS(2) MERGE_BWD_ROWS(3) MERGE_BWD_ROWS(4) MERGE_BWD_ROWS(5) MERGE_BWD_ROWS(6)
 #endif
 
