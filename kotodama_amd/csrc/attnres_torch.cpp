@@ -460,6 +460,13 @@ struct Merge : public torch::autograd::Function<Merge> {
 
 // ---------------------------------------------------------- Python entries --
 
+// How a routing call's result is handed back.
+enum Form : int64_t {
+  kRows = 1,          // the routed rows alone, one query's without its dimension
+  kTuple = 2,         // (out, weights, lse, inv_rms, logits), None where not requested
+  kPlaceholders = 3,  // the same with empty fp32 tensors there (what the op returns)
+};
+
 // The tensor behind an argument of exactly type Tensor or Parameter; undefined
 // for None; false for anything else.
 bool take(PyObject* o, bool none_ok, Tensor* t) {
@@ -493,15 +500,16 @@ bool take(PyObject* o, bool* v) {
   *v = o == Py_True;
   return PyBool_Check(o);
 }
-// out_dtype: a torch.dtype, or None for the promotion of the sources' and the parameters' dtypes
-bool take_dtype(PyObject* o, const Tensor& src, const Tensor& query, const Tensor& gain, at::ScalarType* t) {
+// out_dtype: a torch.dtype; with the rows form and a gain None too, for the promotion of the sources' and
+// the parameters' dtypes (the other forms stand for the op, which takes no None, and the drop-ins need a gain)
+bool take_dtype(PyObject* o, int64_t form, const Tensor& src, const Tensor& query, const Tensor& gain,
+                at::ScalarType* t) {
   if (THPDtype_Check(o)) {
     *t = reinterpret_cast<THPDtype*>(o)->scalar_type;
     return true;
   }
-  if (o != Py_None) return false;
-  *t = at::promote_types(src.scalar_type(), query.scalar_type());
-  if (gain.defined()) *t = at::promote_types(*t, gain.scalar_type());
+  if (o != Py_None || form != kRows || !gain.defined()) return false;
+  *t = at::promote_types(src.scalar_type(), at::promote_types(query.scalar_type(), gain.scalar_type()));
   return true;
 }
 bool take_list(PyObject* o, std::vector<Tensor>* v) {
@@ -538,12 +546,6 @@ PyObject* wrap(const Tensor& t) {
   if (!t.defined()) return none();
   return THPVariable_Wrap(t);
 }
-// How a routing call's result is handed back.
-enum Form : int64_t {
-  kRows = 1,          // the routed rows alone, one query's without its dimension
-  kTuple = 2,         // (out, weights, lse, inv_rms, logits), None where not requested
-  kPlaceholders = 3,  // the same with empty fp32 tensors there (what the op returns)
-};
 PyObject* pack(const Routed& r, int64_t form) {
   if (form == kRows) return wrap(r.out);
   PyObject* tup = PyTuple_New(5);
@@ -567,8 +569,9 @@ PyObject* py_route(PyObject*, PyObject* const* a, Py_ssize_t n) {
   double eps = 0;
   at::ScalarType dt;
   if (n != 11 || !take(a[0], false, &buf) || !take(a[1], &num) || !take(a[2], false, &query) ||
-      !take(a[3], true, &gain) || !take(a[4], &eps) || !take_dtype(a[5], buf, query, gain, &dt) || !take(a[6], &ww) ||
-      !take(a[7], &wl) || !take(a[8], &wa) || !take(a[9], &form) || !unwatched())
+      !take(a[3], true, &gain) || !take(a[4], &eps) || !take(a[9], &form) ||
+      !take_dtype(a[5], form, buf, query, gain, &dt) || !take(a[6], &ww) || !take(a[7], &wl) || !take(a[8], &wa) ||
+      !unwatched())
     return none();
   const bool rec = recorded({&buf, &query, &gain});
   if (rec && (a[10] == Py_None || num < 1 || !no_tangent(buf) || !no_tangent(query) || !no_tangent(gain)))
@@ -601,8 +604,8 @@ PyObject* py_route_list(PyObject*, PyObject* const* a, Py_ssize_t n) {
   int64_t form = 0;
   at::ScalarType dt;
   if (n != 10 || !take_list(a[0], &srcs) || srcs.empty() || !take(a[1], false, &query) || !take(a[2], true, &gain) ||
-      !take(a[3], &eps) || !take_dtype(a[4], srcs[0], query, gain, &dt) || !take(a[5], &ww) || !take(a[6], &wl) ||
-      !take(a[7], &wa) || !take(a[8], &form) || !unwatched())
+      !take(a[3], &eps) || !take(a[8], &form) || !take_dtype(a[4], form, srcs[0], query, gain, &dt) ||
+      !take(a[5], &ww) || !take(a[6], &wl) || !take(a[7], &wa) || !unwatched())
     return none();
   const bool rec = recorded(srcs) || recorded({&query, &gain});
   if (rec) {
@@ -708,7 +711,7 @@ PyObject* py_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
   at::ScalarType dt;
   if (n != 7 || !take_list(a[0], &srcs) || !take(a[1], false, &partial) || !take(a[2], false, &delta) ||
       !take(a[3], false, &query) || !take(a[4], true, &gain) || !take(a[5], &eps) ||
-      !take_dtype(a[6], partial, query, gain, &dt) || !unwatched())
+      !take_dtype(a[6], kTuple, partial, query, gain, &dt) || !unwatched())
     return none();
   const int k = (int)srcs.size();
   srcs.push_back(partial);

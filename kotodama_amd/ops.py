@@ -1206,12 +1206,13 @@ def route_rows(buf, num_sources, query, gain, eps) -> Tensor:
 
 
 def route_list_rows(sources, query, gain, eps) -> Tensor:
-    """:func:`route_rows` over a list of separate blocks."""
+    """:func:`route_rows` over a sequence of separate blocks."""
     if not torch.compiler.is_compiling():
         out = native.route_list(sources, query, gain, eps, None, False, False, False, _ROWS, False)
         if out is not None:
             return out
-    return route_list_call(sources, query, gain, eps, _promoted(sources[0], query, gain))[0].squeeze(0)
+    out_dtype = _promoted(sources[0], query, gain)  # a sequence: an iterator is refused here
+    return route_list_call(list(sources), query, gain, eps, out_dtype)[0].squeeze(0)
 
 
 def _promoted(src: Tensor, query: Tensor, gain: Tensor) -> torch.dtype:

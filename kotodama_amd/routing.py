@@ -64,7 +64,7 @@ def block_attn_res_from_list(sources: Sequence[Tensor], query: Tensor, norm) -> 
     -inf; the padded slots get weight exactly 0, so routing over the list
     itself gives the same result without building the padded buffer.
     """
-    return ops.route_list_rows(list(sources), query, norm.weight, float(norm.eps))
+    return ops.route_list_rows(sources, query, norm.weight, float(norm.eps))
 
 
 def route_weights(buf: Tensor, num_active: int, query: Tensor, norm) -> tuple[Tensor, Tensor, Tensor]:

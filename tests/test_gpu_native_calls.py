@@ -295,3 +295,28 @@ def test_training_loop_equals_the_python_launches(gpu, monkeypatch, d, dtype, re
         assert off or reached <= set(rec.taken), rec.taken
         assert not off or not rec.taken
     _same(*res)
+
+
+def test_calls_the_ops_refuse_stay_refused(gpu):
+    buf, query, gain = _tensors(gpu)
+    rows, blocks = lambda g: kotodama_amd.route_static(buf, query, Norm(g), None, 3), list(buf)
+    for leaves in (False, True):
+        query.requires_grad_(leaves)
+        # no output dtype: only the drop-ins promote one
+        with pytest.raises(RuntimeError, match="out_dtype"):
+            ops.route(buf, 3, query, gain, 1e-5, None, False, False)
+        with pytest.raises(RuntimeError, match="out_dtype"):
+            ops.route_list(blocks, query, gain, 1e-5, None, False, False)
+        for call, src in ((lambda *a: ops.route_call(a[0], 3, *a[1:]), buf), (ops.route_list_call, blocks)):
+            with pytest.raises((TypeError, RuntimeError)):
+                call(src, query, gain, 1e-5, None)
+        # the drop-ins need a gain and a sequence
+        with pytest.raises(AttributeError, match="dtype"):
+            rows(None)
+        with pytest.raises(AttributeError, match="dtype"):
+            kotodama_amd.block_attn_res_from_list(blocks, query, Norm(None))
+        with pytest.raises(TypeError, match="subscriptable"):
+            kotodama_amd.block_attn_res_from_list((b for b in buf), query, Norm(gain))
+    want = rows(gain)
+    for seq in (tuple(blocks), type("Blocks", (list,), {})(blocks)):
+        assert torch.equal(kotodama_amd.block_attn_res_from_list(seq, query, Norm(gain)), want)
